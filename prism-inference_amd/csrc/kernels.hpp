@@ -58,6 +58,11 @@ struct MatvecArgs {
     // Scratch the caller can provide at most (a fixed buffer); kernel choices that need more
     // fall back to ones that need less.
     size_t scratch_cap = ~size_t(0);
+    // Scratch the caller has without growing anything (a fixed buffer, or a stream capture in
+    // progress), and (kActF32) whether the prepared blocks of the call fit its scratch: a path
+    // that needed neither before a batch kernel took its place is kept where they do not.
+    size_t scratch_fit = ~size_t(0);
+    bool act_fit = true;
 };
 
 // Return launch_status() values (0, kLaunchUnsupported, or a hipError_t).
@@ -74,6 +79,9 @@ bool tiled_needs_prepared(const MatvecArgs &a);
 bool tiled_prologue_fits(const MatvecArgs &a);
 // Device scratch a tiled call needs (the lane-ordered activations of a skinny batch).
 size_t tiled_scratch_bytes(const MatvecArgs &a);
+// Whether a call on prepared blocks whose token count the prefill GEMMs take is faster as a
+// skinny batch, with the scratch it has (scratch_fit).
+bool skinny_beats_gemm(const MatvecArgs &a);
 // Whether (kind, cols, rows) can be stored tiled on a device with `cus` compute units
 // (every projection of it then has a tiled kernel), and the native -> tiled repack
 // (the destination must hold tiled_bytes() and be zero-filled beforehand).

@@ -1922,6 +1922,91 @@ __global__ __launch_bounds__(64 * KS) void k_mv_skinny(SkParams p) {
         if (u < p.nu) fold(A);
 #pragma unroll
         for (int v = 0; v < 4; ++v) store(i, 4u * L.s + v, ch[v].result());
+    } else if constexpr (O == Op::PTQ1_PINNED) {
+        // Sixteen lane sums per element and unit (8 dwords of 16-bit pairs) would be 12 KiB of
+        // LDS per wavefront and parity with their four dd_g beside them; the 16 row scales and
+        // the tokens' block scales of a unit take 320 bytes instead, and the fold multiplies
+        // them (the same product).  So eight wavefronts share a block (133 KiB) where two did
+        // (measured at the dispatch).  The four native lanes are independent chains: item
+        // k = (element, lane pair) is one thread's, so the fold runs on every wavefront.
+        __shared__ __attribute__((aligned(16))) uint32_t sums[2][KS][8][256];
+        __shared__ __attribute__((aligned(16))) float4 asl[2][KS][16];
+        __shared__ float dwl[2][KS][16];
+        constexpr int IT = 8 / KS;  // items per thread
+        float Lp[IT][2];
+#pragma unroll
+        for (int k = 0; k < IT; ++k) Lp[k][0] = Lp[k][1] = 0.0f;
+        // Item it: token-major elements, so a batch of few tokens folds on few wavefronts.
+        // Lane l's four sums of a term sit at dwords 4 * (16s + (i + 4s) % 16) (s = l / 16,
+        // i = l % 16): the 16 rows of four tokens, one wavefront's read, then cover all banks.
+        auto slot = [](uint32_t tok, uint32_t r) { return 4u * (16u * (r >> 2) + ((tok + 4u * (r >> 2)) & 15u)) + (r & 3u); };
+        const uint32_t chunks = (p.nu + KS - 1) / KS;
+        auto produce = [&](const SkFrag<O> &f, uint32_t c) {
+            float tv[4][TPU];
+            sk_terms<O>(f, L, pp, tv);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                *reinterpret_cast<float4 *>(&sums[c & 1u][wave][j][slot(i, 4u * L.s)]) =
+                    make_float4(tv[0][j], tv[1][j], tv[2][j], tv[3][j]);
+            if (L.s == 0)
+                asl[c & 1u][wave][i] = make_float4(__uint_as_float(f.as.x), __uint_as_float(f.as.y),
+                                                   __uint_as_float(f.as.z), __uint_as_float(f.as.w));
+            if (i == 0) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) dwl[c & 1u][wave][4u * L.s + v] = h2f(f.dd[v] >> 16);
+            }
+        };
+        auto consume = [&](uint32_t c) {
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                const uint32_t it = threadIdx.x + 64u * KS * k, e = it & 255u, hh = it >> 8;
+                const uint32_t tok = e >> 4, r = e & 15u, at = slot(tok, r);
+                if (tok >= ntok) continue;
+#pragma unroll
+                for (int w = 0; w < KS; ++w) {
+                    if (c * KS + w < p.nu) {
+                        // dot_q8_groups_pinned, src/kernels.rs:1134-1146: per group,
+                        // L[l] = fma(I_l, dd_g, L[l]), dd_g = fl(d_w * A_g.scale).
+                        const float dw = dwl[c & 1u][w][r];
+                        const float4 a4 = asl[c & 1u][w][tok];
+                        const float as[4] = {a4.x, a4.y, a4.z, a4.w};
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const uint32_t pk = sums[c & 1u][w][2 * g + hh][at];
+                            const float dd = dw * as[g];
+                            Lp[k][0] = __builtin_fmaf(static_cast<float>(static_cast<int16_t>(pk & 0xffffu)), dd, Lp[k][0]);
+                            Lp[k][1] = __builtin_fmaf(static_cast<float>(static_cast<int16_t>(pk >> 16)), dd, Lp[k][1]);
+                        }
+                    }
+                }
+            }
+        };
+        SkFrag<O> A, B;
+        uint32_t c = 0;
+        if (wave < p.nu) sk_load<O, SW>(A, L, wave, pp);
+        while (c + 1 < chunks) {
+            const uint32_t u1 = (c + 1) * KS + wave;
+            if (u1 < p.nu) sk_load<O, SW>(B, L, u1, pp);
+            if (c * KS + wave < p.nu) produce(A, c);
+            consume(c);
+            const uint32_t u2 = (c + 2) * KS + wave;
+            if (c + 2 < chunks && u2 < p.nu) sk_load<O, SW>(A, L, u2, pp);
+            if (u1 < p.nu) produce(B, c + 1);
+            consume(c + 1);
+            c += 2;
+        }
+        if (c < chunks) {
+            if (c * KS + wave < p.nu) produce(A, c);
+            consume(c);
+        }
+        // (L0 + L1) + (L2 + L3): the pair sums meet in LDS.
+        __syncthreads();
+        float *pair = reinterpret_cast<float *>(&sums[0][0][0][0]);
+#pragma unroll
+        for (int k = 0; k < IT; ++k) pair[threadIdx.x + 64u * KS * k] = Lp[k][0] + Lp[k][1];
+        __syncthreads();
+        for (uint32_t e = threadIdx.x; e < 256u; e += 64u * KS) store(e >> 4, e & 15u, pair[e] + pair[256u + e]);
     } else {
         // terms[parity][wave][term][element], element e = 4 * lane + v
         __shared__ float terms[2][KS][TPU][256];
@@ -2956,7 +3041,8 @@ int launch_batch(const MatvecArgs &a, const void *act, uint32_t ntok, uint32_t a
     return launch_status();
 }
 
-// Row count from which 2..16 tokens run on the matrix cores (16 rows per wavefront).
+// Row count from which every kind and contract takes the skinny kernel whatever its scratch;
+// below it the rules that led there before (token by token, no scratch) stay the fallback.
 constexpr uint64_t kSkinnyMinRows = 1024;
 
 // The row-tile batch kernel (one wavefront per 64-row tile runs every token's chain, each
@@ -2966,44 +3052,77 @@ bool batch_eligible(const MatvecArgs &a) {
     return a.tokens >= 2 && !a.w2 && a.rows >= kBatchMinRows;
 }
 
-// Whether a skinny batch first copies its activations into lane order (one more launch,
-// then contiguous loads) instead of gathering them from the prepared blocks in every
-// wavefront.  Measured on 2048..151936 rows: the copy pays from 8192 rows or from 5
-// tokens; Q2_K's 256-element units halve its gathers (as TQ2_0's, in the same order), and
-// the copy pays only from 32768 rows.  PQ2 and Q8_0 rows of 12288 inputs or more take it
-// from two tokens (us, gathered / copied: PQ2 5120 x 17408 3 tokens 37.6 / 30.1, 4096 x
-// 14336 4 tokens 26.5 / 24.6; Q8_0 4096 x 14336 2 tokens 31.6 / 28.6); PTQ1 there is mixed
-// (4096 x 14336 4 tokens 31.3 / 38.4, 5120 x 17408 55.4 / 45.9) and keeps the rule above.
+// How a skinny batch runs.  sw: its activations are first copied into lane order (one more
+// launch, then contiguous loads) instead of being gathered from the prepared blocks by every
+// wavefront.  most: 16-token chunks per launch.
+struct SkinnyPlan {
+    bool sw;
+    uint32_t most;
+};
+
+// 16-row blocks of a matrix, one skinny workgroup each.
+uint64_t skinny_blocks(uint64_t rows) { return (rows + kTile - 1) / kTile * 4; }
+
 template <Op O>
-bool skinny_lane_ordered(uint64_t rows, uint64_t cols, uint32_t ntok) {
-    if constexpr (O == Op::Q2K || O == Op::TQ2) return rows >= 32768;
-    if constexpr (O == Op::Q8_0 || kind_of<O>() == kPQ2)
-        if (cols >= 12288) return true;
-    return rows >= 8192 || ntok > 4;
+size_t skinny_chunk_bytes(const MatvecArgs &a) {
+    return a.cols / unit_weights<O>() * 64u * (sk_lane_bytes<O>() + 4u);
 }
 
-// 16-token chunks per skinny launch: the chunks run side by side (grid y), each a batch
-// of its own, so a launch of up to kSkChunks * 16 tokens fills the chip where one chunk
-// leaves it latency-bound.  Four chunks keep the lane-ordered copies under 10 MB at
-// 65536 inputs.
-constexpr uint32_t kSkChunks = 4;
+// The copy costs a launch; the gathers cost every wavefront scattered loads, more with more
+// tokens.  Measured, f32 input (us, gathered / copied): Q8_0 pays for the copy from 5 tokens (850
+// x 5120, 7 tokens 14.7 / 12.6).  The others take it from 9 (7 tokens: PTQ1 2048 x 2048 9.4 /
+// 12.2, pinned 10.7 / 13.8, PQ2 4096 x 4096 10.0 / 10.8, TQ1_0 9.5 / 10.4; 16 tokens: PTQ1 850 x
+// 5120 20.9 / 17.8, PQ2 12.2 / 11.7, TQ1_0 12.4 / 11.4), from 5 where many units are gathered
+// (7 tokens: PTQ1 6144 x 5120 24.4 / 20.0, pinned 4302 x 10752 48.3 / 53.9, TQ1_0 1100 x 12800
+// 17.9 / 16.5), and not at all on short PTQ1 rows of few blocks (850 x 2560, 64 tokens 13.5 /
+// 19.6, pinned 15.3 / 21.8; 2048 x 2048, 64 tokens 16.7 / 18.3, 96 tokens equal).  Every format
+// takes it from 8192 rows, but Q2_K's and TQ2_0's 256-element units halve the gathers (32768 x
+// 2048 Q2_K, 7 tokens 10.9 / 13.5; 40000 x 5120, 16 tokens 31.9 / 29.3).  PQ2 and Q8_0 rows of
+// 12288 inputs or more take it from two tokens (PQ2 5120 x 17408 3 tokens 37.6 / 30.1, 4096 x
+// 14336 4 tokens 26.5 / 24.6; Q8_0 4096 x 14336 2 tokens 31.6 / 28.6).
+template <Op O>
+SkinnyPlan skinny_plan(const MatvecArgs &a) {
+    const uint64_t nu = a.cols / unit_weights<O>(), blocks = skinny_blocks(a.rows);
+    const uint64_t chunks = (a.tokens + kBatchMax - 1) / kBatchMax;
+    SkinnyPlan pl;
+    if constexpr (O == Op::Q2K || O == Op::TQ2) {
+        pl.sw = a.rows >= 65536 || (a.rows >= 32768 && a.tokens > 8 && a.cols >= 4096);
+    } else if (a.rows >= 8192 || ((O == Op::Q8_0 || kind_of<O>() == kPQ2) && a.cols >= 12288)) {
+        pl.sw = true;
+    } else if (O == Op::Q8_0 || a.tokens <= 4) {
+        pl.sw = a.tokens > 4;
+    } else if (a.tokens <= 8) {
+        pl.sw = O == Op::TQ1 ? nu > 24 : blocks * nu > (O == Op::PTQ1_PINNED ? 96ull : 32ull) * a.cus;
+    } else {
+        pl.sw = !(kind_of<O>() == kPTQ1 && nu <= 24 && a.rows < 4096 && blocks * chunks * nu <= 48ull * a.cus);
+    }
+    // The chunks of a launch run side by side (grid y), each a batch of its own, so several fill
+    // the chip where one leaves it latency-bound (PQ2 1003 x 8320, 338 tokens, us: 4 / 8 / 16 /
+    // 24 chunks a launch 82 / 53 / 45 / 34).  Thirty-two keep the lane-ordered copies of rows of
+    // up to 17408 inputs under 12 MB; a scratch that holds fewer takes fewer.
+    pl.most = 32;
+    if (pl.sw) {
+        const uint64_t room = a.scratch_fit / skinny_chunk_bytes<O>(a);
+        if (pl.most > room) pl.most = room < 4 ? 4u : static_cast<uint32_t>(room);
+        if (a.rows < kSkinnyMinRows && (chunks < pl.most ? chunks : pl.most) > room) pl.sw = false;
+    }
+    return pl;
+}
 
 template <Op O>
 size_t skinny_scratch(const MatvecArgs &a) {
-    if (!skinny_lane_ordered<O>(a.rows, a.cols, a.tokens < kBatchMax ? a.tokens : kBatchMax)) return 0;
-    const uint64_t nu = a.cols / unit_weights<O>();
+    const SkinnyPlan pl = skinny_plan<O>(a);
     const uint64_t chunks = (a.tokens + kBatchMax - 1) / kBatchMax;
-    return nu * 64u * (sk_lane_bytes<O>() + 4u) * (chunks < kSkChunks ? chunks : kSkChunks);
+    return pl.sw ? skinny_chunk_bytes<O>(a) * (chunks < pl.most ? chunks : pl.most) : 0;
 }
 
-// ntok: up to kSkChunks * 16 tokens, one chunk of 16 per grid row.
+// One launch: ntok tokens of the batch `a`, up to pl.most chunks of 16, one per grid row.
 template <Op O>
-int launch_skinny(const MatvecArgs &a, const void *act, uint32_t ntok, uint32_t act_stride, float *out,
-                  const float *residual) {
+int launch_skinny(const MatvecArgs &a, const SkinnyPlan &pl, const void *act, uint32_t ntok, uint32_t act_stride,
+                  float *out, const float *residual) {
     const uint32_t chunks = (ntok + kBatchMax - 1) / kBatchMax;
-    if (chunks > kSkChunks) return -2;
-    const bool sw = skinny_lane_ordered<O>(a.rows, a.cols, ntok < kBatchMax ? ntok : kBatchMax);
-    if (sw && (!a.scratch || a.scratch_bytes < skinny_scratch<O>(a))) return -2;
+    const bool sw = pl.sw;
+    if (sw && (!a.scratch || a.scratch_bytes < skinny_chunk_bytes<O>(a) * chunks)) return -2;
     const uint32_t nu = static_cast<uint32_t>(a.cols / unit_weights<O>());
     const uint32_t sw_chunk = nu * 64u * (sk_lane_bytes<O>() + 4u);
     if (sw) {
@@ -3022,23 +3141,23 @@ int launch_skinny(const MatvecArgs &a, const void *act, uint32_t ntok, uint32_t 
     p.rows = static_cast<uint32_t>(a.rows);
     p.nu = nu;
     p.ntok = ntok;
-    const uint64_t tiles = (a.rows + kTile - 1) / kTile;
-    // Wavefronts per 16-row block: enough to give the chip about eight per SIMD.
-    const uint64_t blocks = tiles * 4;
-    const uint64_t want = 32ull * a.cus;
-    int ks = blocks >= want ? 1 : blocks * 2 >= want ? 2 : blocks * 4 >= want ? 4 : 8;
-    // The LDS terms buffer is 2 * KS * terms * 1 KiB: pinned PTQ1's twelve terms per
-    // element cap it at two wavefronts per block (48 KiB).
-    constexpr int kMaxKs = sk_terms_per_unit<O>() > 8 ? 2 : 8;
-    if (ks > kMaxKs) ks = kMaxKs;
+    // Wavefronts per 16-row block.  One keeps its chains in registers and needs no LDS or
+    // barrier; eight share a block's units where blocks and chunks leave the chip idle.
+    // Measured (us, wavefronts 1 / 2 / 4 / 8): Q2_K 12288 x 4096 7 tokens (three workgroups per
+    // CU) 12.1 / 12.2 / 10.4 / 10.7, PQ2 20.3 / 18.5 / 13.9 / 12.8; 32768 x 2048 (eight) Q2_K
+    // 13.9 / 14.6 / 14.4 / 15.6, Q8_0 17.5 / 19.4 / 20.0 / 21.4; 40000 x 5120 16 tokens (ten) Q2_K
+    // 31.9 / - / 29.4 / -, TQ2_0 29.8 / - / 26.7 / -; from sixteen one is ahead.  Pinned PTQ1's fold
+    // is its larger part, and its terms leave one workgroup of eight to a CU: 512 x 2048 7 tokens
+    // 16.1 / 16.7 / 12.4 / 10.6, 6144 x 2048 (1.5 per CU) 16.1 / 18.4 / 15.5 / 17.5, 9000 x 4096
+    // (2.2) 28.3 / 35.3 / 36.7 / 38.8.
+    const uint64_t blocks = skinny_blocks(a.rows), wgs = blocks * chunks;
+    const int ks = O == Op::PTQ1_PINNED ? (wgs >= 2ull * a.cus ? 1 : wgs > a.cus ? 4 : 8)
+                                        : (wgs >= 16ull * a.cus ? 1 : wgs >= 8ull * a.cus ? 4 : 8);
     const dim3 grid(static_cast<uint32_t>(blocks), chunks), block(64 * ks);
     auto go = [&]<bool SWv>() {
         if (ks == 1) hipLaunchKernelGGL((k_mv_skinny<O, SWv, 1>), grid, block, 0, a.stream, p);
-        else if (ks == 2) hipLaunchKernelGGL((k_mv_skinny<O, SWv, 2>), grid, block, 0, a.stream, p);
-        else if constexpr (kMaxKs >= 8) {
-            if (ks == 4) hipLaunchKernelGGL((k_mv_skinny<O, SWv, 4>), grid, block, 0, a.stream, p);
-            else hipLaunchKernelGGL((k_mv_skinny<O, SWv, 8>), grid, block, 0, a.stream, p);
-        }
+        else if (ks == 4) hipLaunchKernelGGL((k_mv_skinny<O, SWv, 4>), grid, block, 0, a.stream, p);
+        else hipLaunchKernelGGL((k_mv_skinny<O, SWv, 8>), grid, block, 0, a.stream, p);
     };
     if (sw)
         go.template operator()<true>();
@@ -3247,6 +3366,37 @@ int launch_splitk(const MatvecArgs &a, uint32_t act_stride) {
     return launch_status();
 }
 
+// Matrices of few rows leave the GEMMs' 128-row workgroups on a fraction of the CUs, and each
+// walks every unit of its rows: their time barely depends on the tokens.  The skinny kernel
+// spreads the same work over 16-row x 16-token workgroups of eight wavefronts, so it is ahead
+// until its grid W = 16-row blocks x token chunks fills the chip (one launch: 512 tokens).
+// Measured (f32 input with its quantization, us, GEMM / skinny): Q2_K 520 x 5120 256 tokens (W
+// 576) 30 / 16, 2048 x 5120 256 (2048) 31 / 27, 400 (3200) 33 / 42; Q8_0 1100 x 10752 160 (720)
+// 89 / 38, 4096 x 5120 160 (2560) 47 / 38, 256 (4096) 49 / 53; PQ2 1100 x 10752 256 (1152) 45 /
+// 38, 3000 x 2048 100 (1316) 14 / 14, 160 (1880) 15 / 16; TQ1_0 1500 x 5120 256 (1536) 27 / 27,
+// 400 (2400) 30 / 34; TQ2_0 1500 x 5120 256 24 / 23, 400 27 / 32.  The PTQ1 GEMMs take longer
+// per unit of a row, so there the line grows with the units (16 / 40 / 84 of them): pinned 800
+// rows 256 tokens (832) 31 / 30, 67 / 44, 133 / 103; 2048 rows 160 (1280) 31 / 36, 67 / 60, 133 /
+// 102; 3000 rows 256 (3008) 31 / 45, 68 / 79, 133 / 141; source 1100 rows 256 (1152) 23 / 28, 45
+// / 38, 87 / 54; 4096 rows 160 (2560) 23 / 33, 46 / 49, 88 / 78, and a little lower up to 128
+// tokens, where the block-split kernel runs (2048 rows 100 tokens (896) 19 / 26, 35 / 34, 66 /
+// 48).
+bool skinny_beats_gemm(const MatvecArgs &a) {
+    if (a.act_format == kActF32 || a.tokens < 2 || a.tokens > 512 || a.w2 || a.residual || a.tile_best) return false;
+    const uint64_t w = skinny_blocks(a.rows) * ((a.tokens + kBatchMax - 1) / kBatchMax);
+    return dispatch(a, [&]<Op O>() {
+               const uint64_t nu = a.cols / unit_weights<O>();
+               uint64_t most;  // per 256 CUs
+               if constexpr (O == Op::PTQ1_PINNED) most = nu < 44 ? 600 + 25 * nu : 1700;
+               else if constexpr (kind_of<O>() == kPTQ1) most = nu < 50 ? (a.tokens > 128 ? 40 : 30) * nu : 2000;
+               else if constexpr (O == Op::Q2K) most = 2048;
+               else if constexpr (O == Op::Q8_0) most = 2560;
+               else if constexpr (kind_of<O>() == kPQ2) most = 1300;
+               else most = 1500;
+               return w * 256 <= most * a.cus && skinny_scratch<O>(a) <= a.scratch_fit ? 1 : 0;
+           }) == 1;
+}
+
 // Prepared activations of many tokens on the prefill GEMMs, from the token counts at which
 // they beat the skinny kernel for f32 input: Q8_K blocks for Q2_K, PQ2, TQ1_0 and TQ2_0, Q8_0
 // blocks for Q8_0 (int8 GEMM, prefill_k.hip) and PTQ1 in either order (f16 GEMM,
@@ -3258,14 +3408,20 @@ bool gemm_eligible(const MatvecArgs &a) {
     const bool fits = a.act_format == kActQ8K
                           ? a.kind == kQ2_K || a.kind == kPQ2 || a.kind == kTQ1_0 || a.kind == kTQ2_0
                           : a.kind == kQ8_0 || a.kind == kPTQ1;
-    return fits && prefill_supported(a.kind, a.cols, a.rows, a.pinned, a.tokens) &&
+    return fits && prefill_supported(a.kind, a.cols, a.rows, a.pinned, a.tokens) && !skinny_beats_gemm(a) &&
            prefill_scratch_bytes(a.kind, a.cols, a.tokens) <= a.scratch_cap;
 }
 
 bool skinny_eligible(const MatvecArgs &a) {
-    if (a.tokens < 2 || a.w2 || a.rows < kSkinnyMinRows || lut_batch_eligible(a) || quad_eligible(a) ||
-        quad_split_eligible(a))
-        return false;
+    if (a.tokens < 2 || a.w2 || lut_batch_eligible(a) || quad_eligible(a) || quad_split_eligible(a)) return false;
+    if (a.rows < kSkinnyMinRows && a.act_format == kActF32) {
+        // f32 input ran token by token here, each launch quantizing in its prologue: two
+        // source-order PTQ1 tokens of rows too short for split-K stay there (us, token by token /
+        // quantizer + skinny: 512 x 2048 7.2 / 7.7, four tokens 15.4 / 8.4; the other formats
+        // gain from two, Q2_K 850 x 5120 12.5 / 7.7, pinned PTQ1 23.1 / 15.0; split-K 700 x 15232
+        // 19.0 / 15.1), and so does a call whose prepared blocks do not fit the caller's scratch.
+        if (!a.act_fit || (a.tokens == 2 && a.kind == kPTQ1 && !a.pinned && a.cols < kSplitKMinUnits * 128)) return false;
+    }
     // Pinned PTQ1 (four masked MFMAs per group) and TQ1_0 / TQ2_0 (digits decoded for 16
     // rows per wavefront) on large matrices: up to four tokens the row-tile batch kernel is
     // faster (151936x4096 x 4: pinned PTQ1 148 against 165 us, TQ2_0 56.8 against 61.3, TQ1_0
@@ -3289,6 +3445,9 @@ bool skinny_eligible(const MatvecArgs &a) {
 bool token_by_token(const MatvecArgs &a) {
     const uint64_t tiles = (a.rows + kTile - 1) / kTile;
     if (a.w2 || tiles >= 2ull * a.cus || a.cols < 6144 || (a.kind != kPTQ1 && a.kind != kPQ2)) return false;
+    // Pinned PTQ1 takes the skinny kernel (us, two tokens, token by token / skinny: 4302 x
+    // 10752 52.9 / 41.6, 5120 x 6144 34.1 / 26.2, 1567 x 15232 49.0 / 32.3).
+    if (a.kind == kPTQ1 && a.pinned && a.act_format == kActQ8) return false;
     return a.tokens == 2 || (a.tokens == 3 && a.kind == kPTQ1 && a.cols >= 12288);
 }
 
@@ -3316,17 +3475,19 @@ int launch_matvec_tiled(const MatvecArgs &a) {
     if (batched && lut_batch_eligible(a))
         return dispatch(a, [&]<Op O>() { return launch_lut_batch<O>(a, static_cast<uint32_t>(in_stride)); });
     if (batched && skinny_eligible(a)) {
-        for (uint32_t tok = 0; tok < a.tokens; tok += kSkChunks * kBatchMax) {
-            const uint32_t n = a.tokens - tok < kSkChunks * kBatchMax ? a.tokens - tok : kSkChunks * kBatchMax;
-            const void *act = static_cast<const uint8_t *>(a.act) + in_stride * tok;
-            float *out = a.out + a.rows * tok;
-            const float *res = a.residual ? a.residual + a.rows * tok : nullptr;
-            const int rc = dispatch(a, [&]<Op O>() {
-                return launch_skinny<O>(a, act, n, static_cast<uint32_t>(in_stride), out, res);
-            });
-            if (rc) return rc;
-        }
-        return 0;
+        return dispatch(a, [&]<Op O>() {
+            const SkinnyPlan pl = skinny_plan<O>(a);
+            const uint32_t most = pl.most * kBatchMax;
+            for (uint32_t tok = 0; tok < a.tokens; tok += most) {
+                const uint32_t n = a.tokens - tok < most ? a.tokens - tok : most;
+                const void *act = static_cast<const uint8_t *>(a.act) + in_stride * tok;
+                float *out = a.out + a.rows * tok;
+                const float *res = a.residual ? a.residual + a.rows * tok : nullptr;
+                const int rc = launch_skinny<O>(a, pl, act, n, static_cast<uint32_t>(in_stride), out, res);
+                if (rc) return rc;
+            }
+            return 0;
+        });
     }
     if (batched && batch_eligible(a)) {
         for (uint32_t tok = 0; tok < a.tokens; tok += kBatchMax) {

@@ -19,13 +19,30 @@ namespace {
 // has the last word: its own thresholds per kind, contract and matrix size).
 constexpr uint32_t kPrefillMinTokens = 16;
 
+// Whether a projection of f32 input runs as a tiled-prefill GEMM: its token count reaches the
+// GEMM's and the skinny batch is not faster, or its blocks (in `role`) and lane-ordered copy
+// would not fit a fixed or captured scratch.
+bool gemm_path(prism_hip_ctx *c, const Weight &w, uint32_t tokens, int pinned, const Scratch *sc, const DevBuf &role,
+               const float *residual) {
+    if (!w.tiled || tokens < kPrefillMinTokens || !prefill_supported(w.kind, w.cols, w.rows, pinned, tokens)) return false;
+    const int contract = contract_for(w.kind, w.cols, pinned);
+    MatvecArgs a = matvec_args(c, w, contract == 0 ? kActQ8K : kActQ8, nullptr, tokens, pinned, nullptr, c->stream);
+    const size_t act = (act_bytes(contract, w.cols, tokens) + 255) & ~size_t(255);
+    a.residual = residual;
+    if (!skinny_beats_gemm(a)) return true;
+    if (act > scratch_room(c, sc, role, act)) return true;
+    a.scratch_fit = scratch_room(c, sc, c->sk, tiled_scratch_bytes(a));
+    if (sc && sc->base) a.scratch_fit -= act;  // one region holds both
+    return !skinny_beats_gemm(a);
+}
+
 // Quantize device floats with the contract matvec_into would use, then project.  `role`
 // is the grow-mode buffer of the quantized activation; sc == nullptr selects grow mode.
 int project_f32_dev(prism_hip_ctx *c, const Weight &w, const float *x, uint32_t tokens, int pinned, float *out,
                     DevBuf &role, hipStream_t s, const float *residual = nullptr, Scratch *sc = nullptr) {
     Scratch grow{c};
     Scratch &scr = sc ? *sc : grow;
-    if (w.tiled && tokens >= kPrefillMinTokens && prefill_supported(w.kind, w.cols, w.rows, pinned, tokens)) {
+    if (gemm_path(c, w, tokens, pinned, sc, role, residual)) {
         void *pre = nullptr;
         int rc = scr.get(c->pre, prefill_scratch_bytes(w.kind, w.cols, tokens), &pre);
         if (rc) return rc;
@@ -39,6 +56,10 @@ int project_f32_dev(prism_hip_ctx *c, const Weight &w, const float *x, uint32_t 
     }
     if (w.tiled) {
         MatvecArgs a = f32_args(c, w, x, tokens, pinned, out, residual, s);
+        if (tokens > 1) {
+            const size_t act = act_bytes(contract_for(w.kind, w.cols, pinned), w.cols, tokens);
+            a.act_fit = act <= scratch_room(c, sc, role, act);
+        }
         if (!tiled_needs_prepared(a)) return run_matvec(c, a, true, &scr);
     }
     const int contract = contract_for(w.kind, w.cols, pinned);
@@ -235,7 +256,7 @@ int group_tokens_impl(prism_hip_ctx *c, const Weight *const *w, uint32_t n, cons
     bool prepared = false;
     for (uint32_t i = 0; i < n; ++i) {
         const Weight &wi = *w[i];
-        bool own = wi.tiled && tokens >= kPrefillMinTokens && prefill_supported(wi.kind, wi.cols, wi.rows, pinned, tokens);
+        bool own = gemm_path(c, wi, tokens, pinned, nullptr, c->act, nullptr);
         if (!own && wi.tiled && tokens == 1) own = !tiled_needs_prepared(f32_args(c, wi, x, 1, pinned, outs[i], nullptr, s));
         int rc;
         if (own) {

@@ -303,15 +303,31 @@ inline MatvecArgs matvec_args(prism_hip_ctx *c, const Weight &w, int act_format,
     return a;
 }
 
+// Scratch of a role that a call can have without growing it: the rest of a fixed region, or
+// the buffer as it is while the stream is being captured; otherwise no limit.  A buffer that
+// already holds `need` bytes is not asked about (the capture query costs about 0.4 us).
+inline size_t scratch_room(prism_hip_ctx *c, const Scratch *sc, const DevBuf &role, size_t need) {
+    if (sc && sc->base) {
+        const size_t at = (sc->used + 255) & ~size_t(255);
+        return at < sc->cap ? sc->cap - at : 0;
+    }
+    if (need <= role.cap) return ~size_t(0);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool capturing = hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+    return capturing ? role.cap : ~size_t(0);
+}
+
 // sc == nullptr: the context's grow-only buffers.
 inline int run_matvec(prism_hip_ctx *c, const MatvecArgs &args, bool tiled, Scratch *sc = nullptr) {
     MatvecArgs a = args;
     if (tiled) {
-        if (sc && sc->base) {  // a fixed buffer: what is left of it bounds the kernel choice
-            const size_t at = (sc->used + 255) & ~size_t(255);
-            a.scratch_cap = at < sc->cap ? sc->cap - at : 0;
+        // A fixed buffer: what is left of it bounds the kernel choice.
+        if (sc && sc->base) a.scratch_cap = a.scratch_fit = scratch_room(c, sc, c->sk, 0);
+        size_t need = tiled_scratch_bytes(a);
+        if (need && !(sc && sc->base)) {
+            a.scratch_fit = scratch_room(c, sc, c->sk, need);
+            if (a.scratch_fit < need) need = tiled_scratch_bytes(a);
         }
-        const size_t need = tiled_scratch_bytes(a);
         if (need) {
             Scratch grow{c};
             const int e = (sc ? *sc : grow).get(c->sk, need, &a.scratch, &a.scratch_bytes);
