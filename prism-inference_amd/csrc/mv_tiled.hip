@@ -620,6 +620,30 @@ struct Chain {
     }
 };
 
+// One native lane's step of the pinned PTQ1 chain (dot_q8_groups_pinned, src/kernels.rs:1134-1146)
+// over group g of a unit: pk holds the lane sums of lanes l & ~1 and l | 1, dd = fl(d_w * A_g.scale).
+__device__ __forceinline__ float pinned_lane_step(uint32_t pk, uint32_t l, float dd, float L) {
+    return __builtin_fmaf(static_cast<float>(static_cast<int16_t>(pk >> (16u * (l & 1u)))), dd, L);
+}
+// (L0 + L1) + (L2 + L3) over the four lanes of a quad.
+__device__ __forceinline__ float pinned_quad_sum(float L) {
+    L = L + dpp_f<kDppXor1>(L);
+    return L + dpp_f<kDppXor2>(L);
+}
+// Native lane l's chain over a row's nu units (terms t of tpu floats a unit, prepared blocks
+// `act`), summed over the quad's four lanes.
+__device__ __forceinline__ float pinned_lane_sum(const float *t, uint32_t tpu, const void *act, uint32_t nu, uint32_t l) {
+    const Q8Block *b = static_cast<const Q8Block *>(act);
+    float L = 0.0f;
+    // Few threads run this, so their LDS reads are issued several units ahead of the chain.
+#pragma unroll 4
+    for (uint32_t u = 0; u < nu; ++u, t += tpu, b += 4) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) L = pinned_lane_step(__float_as_uint(t[2 * g + (l >> 1)]), l, t[8] * b[g].scale, L);
+    }
+    return pinned_quad_sum(L);
+}
+
 // Kernel parameters (passed by value).
 struct MvParams {
     const uint8_t *w[2];  // tiled weights; w[1] is the FFN up matrix when NMAT == 2
@@ -1009,6 +1033,122 @@ __global__ __launch_bounds__(kLutThreads) void k_mv_rows_lut(MvParams p, const v
                 }
             }
         }
+    }
+}
+
+// Rows of any length, one workgroup of sixteen wavefronts per tile (or walking several): the
+// wavefronts take the workgroup's units sixteen at a time, in order, and leave their terms in
+// one of two LDS buffers, which the folding wavefronts read after the barrier while all sixteen
+// compute the next sixteen.  So a tile keeps sixteen wavefronts busy whatever its row length,
+// where the spread form needs every unit's terms in LDS and the whole form gives a tile one
+// wavefront.  Pinned PTQ1 folds on four wavefronts, one native lane of a row per thread (its
+// fold is as long as its dots); the single-term orders on the first.
+// kStreamRow: floats per term, the 64 rows and (pinned) 16 of padding, so that the two packed
+// words a wavefront's quads read lie in different banks.  The table, the buffers and the block
+// scales of 256 units take 157 KiB.
+constexpr uint32_t kStreamMaxUnits = 256;
+template <Op O>
+constexpr uint32_t kStreamRow = O == Op::PTQ1_PINNED ? 80 : 64;
+template <Op O>
+constexpr uint32_t stream_lds() {
+    return (2 * kLutWaves * terms_per_unit<O>() * kStreamRow<O> + (O == Op::PTQ1_PINNED ? 4 * kStreamMaxUnits : 0)) *
+           static_cast<uint32_t>(sizeof(float));
+}
+template <Op O>
+__global__ __launch_bounds__(kLutThreads) void k_mv_stream_lut(MvParams p, const void *__restrict__ act) {
+    extern __shared__ __attribute__((aligned(16))) float stream_terms[];
+    constexpr uint32_t UB = unit_bytes<O>(), TPU = terms_per_unit<O>(), SR = kStreamRow<O>;
+    const uint32_t lane = threadIdx.x & 63u, lbase = 8u * (lane & 31u);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tiles = (p.rows + kTile - 1) / kTile, nu = p.nu, row_bytes = nu * UB;
+    // The workgroup's items: unit i % nu of its tile i / nu (tile blockIdx.x + gridDim.x * k).
+    const uint32_t mine = (tiles - blockIdx.x + gridDim.x - 1) / gridDim.x, items = mine * nu;  // blockIdx.x < tiles
+    auto tile_at = [&](uint32_t k) { return blockIdx.x + gridDim.x * k; };
+    auto rows_of = [&](uint32_t tile) {
+        const uint32_t left = p.rows - tile * kTile;
+        return left < kTile ? left : kTile;
+    };
+    uint32_t ik = wave / nu, iu = wave - ik * nu;  // this wavefront's next item
+    auto load = [&](Raw<O> &w, uint32_t &u) {
+        const uint32_t tile = tile_at(ik), trp = (rows_of(tile) + 7u) & ~7u;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.w[0] + static_cast<size_t>(tile) * kTile * row_bytes, trp * row_bytes);
+        load_unit<O>(w, rs, iu * trp * UB, trp, lane);
+        u = iu;
+        for (iu += kLutWaves; iu >= nu; iu -= nu) ++ik;
+    };
+    Raw<O> A, B;
+    uint32_t ua = 0, ub = 0;
+    if (wave < items) load(A, ua);
+    ptq1_lut_fill(threadIdx.x, blockDim.x);
+    float4 *scl = reinterpret_cast<float4 *>(stream_terms + 2 * kLutWaves * TPU * SR);
+    if constexpr (O == Op::PTQ1_PINNED) {
+        const Q8Block *b = static_cast<const Q8Block *>(act);
+        for (uint32_t u = threadIdx.x; u < nu; u += kLutThreads)
+            scl[u] = make_float4(b[4 * u].scale, b[4 * u + 1].scale, b[4 * u + 2].scale, b[4 * u + 3].scale);
+    }
+    __syncthreads();
+    auto produce = [&](const Raw<O> &w, uint32_t u, uint32_t c) {
+        float t[TPU];
+        unit_terms<O, true>(w, act, u, t, lbase);
+        float *dst = stream_terms + ((c & 1u) * kLutWaves + wave) * TPU * SR + lane;
+#pragma unroll
+        for (uint32_t j = 0; j < TPU; ++j) dst[j * SR] = t[j];
+    };
+    // The fold: row fr of the tile (pinned: 16 rows and four native lanes per wavefront).
+    constexpr uint32_t kFoldWaves = O == Op::PTQ1_PINNED ? 4 : 1;
+    const uint32_t fr = O == Op::PTQ1_PINNED ? 16u * wave + (lane >> 2) : lane, fl = lane & 3u;
+    float o = 0.0f;
+    uint32_t fu = 0, fk = 0;  // the next unit to fold and its tile
+    auto fold = [&](uint32_t c) {
+        const uint32_t n = items - c * kLutWaves < kLutWaves ? items - c * kLutWaves : kLutWaves;
+        const float *src = stream_terms + (c & 1u) * kLutWaves * TPU * SR + fr;
+        auto one = [&](uint32_t w) {
+            const float *t = src + w * TPU * SR;
+            if constexpr (O == Op::PTQ1_PINNED) {
+                const float4 s4 = scl[fu];
+                const float dw = t[8 * SR], sc[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+                for (uint32_t g = 0; g < 4; ++g)
+                    o = pinned_lane_step(__float_as_uint(t[(2 * g + (fl >> 1)) * SR]), fl, dw * sc[g], o);
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < TPU; ++j) o = o + t[j * SR];
+            }
+            if (++fu == nu) {  // uniform: the tile's last unit
+                float v = o;
+                if constexpr (O == Op::PTQ1_PINNED) v = pinned_quad_sum(o);
+                const uint32_t tile = tile_at(fk);
+                if (fr < rows_of(tile) && (O != Op::PTQ1_PINNED || fl == 0)) {
+                    const size_t row = static_cast<size_t>(tile) * kTile + fr;
+                    if (p.residual) v = v + p.residual[row];
+                    p.out[row] = v;
+                    if (!finite(v)) raise_error(p.err, kErrNonfinite);
+                }
+                o = 0.0f;
+                fu = 0;
+                ++fk;
+            }
+        };
+        if (n == kLutWaves) {
+#pragma unroll 4
+            for (uint32_t w = 0; w < kLutWaves; ++w) one(w);
+        } else {
+            for (uint32_t w = 0; w < n; ++w) one(w);
+        }
+    };
+    // Round c: items 16c .. 16c + 15; its terms are folded after its barrier, and the buffer is
+    // written again two rounds later, behind the next barrier.
+    const uint32_t rounds = (items + kLutWaves - 1) / kLutWaves;
+    for (uint32_t c = 0; c < rounds; c += 2) {
+        if ((c + 1) * kLutWaves + wave < items) load(B, ub);
+        if (c * kLutWaves + wave < items) produce(A, ua, c);
+        __syncthreads();
+        if (wave < kFoldWaves) fold(c);
+        if (c + 1 == rounds) break;
+        if ((c + 2) * kLutWaves + wave < items) load(A, ua);
+        if ((c + 1) * kLutWaves + wave < items) produce(B, ub, c + 1);
+        __syncthreads();
+        if (wave < kFoldWaves) fold(c + 1);
     }
 }
 
@@ -2281,7 +2421,18 @@ __global__ __launch_bounds__(kSplitMaxThreads) void k_mv_split(MvParams p) {
 
     // ---- fold in unit order and epilogue ---------------------------------------------
     float o = 0.0f;
-    if (folder) {
+    if constexpr (O == Op::PTQ1_PINNED) {
+        // The four native lanes of a row are independent chains, four adjacent threads run
+        // them: one thread per row spent 16 conversions and FMAs a unit where the dots took a
+        // few (2048 x 17408: 28.5 us against 9.1 in the source order).
+        const float *all = reinterpret_cast<const float *>(smem + abytes);
+        for (uint32_t it = threadIdx.x; it < NMAT * rw * 4u; it += blockDim.x) {
+            const float v = pinned_lane_sum(all + (it >> 2) * stride, TPU, act, nu, it & 3u);
+            if ((it & 3u) == 0) res[it >> 2] = v;
+        }
+        __syncthreads();
+        if (folder) o = res[mat * rw + lane];
+    } else if (folder) {
         Chain<O> ch;
         const float *t = terms + lane * stride;
         for (uint32_t v = 0; v < nu; ++v) ch.fold(t + v * TPU, act, v);
@@ -2294,8 +2445,10 @@ __global__ __launch_bounds__(kSplitMaxThreads) void k_mv_split(MvParams p) {
             if (!finite(o)) raise_error(p.err, kErrNonfinite);
         }
     } else {
-        if (folder) res[mat * rw + lane] = o;
-        __syncthreads();
+        if constexpr (O != Op::PTQ1_PINNED) {
+            if (folder) res[mat * rw + lane] = o;
+            __syncthreads();
+        }
         if (wave == 0) {
             const bool own = lane < rw && valid;
             float h = 0.0f;
@@ -2793,6 +2946,39 @@ bool plan_split(uint64_t rows, uint32_t nu, uint32_t cols, bool quant, uint32_t 
     return pl->lds <= kSplitLds;
 }
 
+// Whether a one-token projection of prepared blocks takes the stream form of the table kernel.
+// Measured (f32 input with its quantization, us, the former kernel / stream; 25 / 40 / 80 / 136
+// units a row at 3200 / 5120 / 10240 / 17408 inputs).  Pinned: 12288 rows 11.8 / 10.8, 15.2 /
+// 13.2, 28.7 / 18.9, 67.7 / 29.7 (2048 inputs 7.0 / 9.0); 20000 rows 25.4 / 15.1, 37.4 / 19.3,
+// 64.2 / 32.8, 106 / 52.8; 65536 rows 26.8 / 23.8, 39.7 / 32.4 (2048 inputs 18.5 / 16.7); 90000
+// rows 27.5 / 31.6, 40.2 / 44.9: its workgroups walk their tiles one by one, where sixteen
+// wavefronts walk sixteen, so beyond four tiles per CU whole tiles win.  Source: 12288 rows 10.8
+// / 10.9, 17.1 / 14.3, 28.4 / 22.9; the spread and split forms hold rows of up to 64 units
+// (20000 rows 9.8 / 11.7, 11.8 / 13.8) and past them whole tiles took 58.5 / 23.7, 96.4 / 37.3;
+// 40000 rows x 10240 60.4 / 33.1, about eight microseconds more per tile and CU.
+// Below half a tile per CU the split kernel is ahead (pinned 8000 x 10240 16.7 / 18.6, 2048 x
+// 17408 15.8 / 27.4) but for the longest pinned rows (4096 x 17408 29.9 / 27.3, 8000 x 17408
+// 39.5 / 27.8: every one of its workgroups stages the whole input).
+template <Op O>
+bool takes_stream(uint64_t tiles, uint32_t nu, uint32_t cus) {
+    if constexpr (kind_of<O>() != kPTQ1) return false;
+    if (nu > kStreamMaxUnits) return false;
+    if (2 * tiles <= cus) return O == Op::PTQ1_PINNED && nu >= 128 && 6 * tiles > cus;
+    if constexpr (O == Op::PTQ1_PINNED) return tiles <= 4ull * cus && nu >= (tiles > 2ull * cus ? 16u : 25u);
+    return tiles < cus ? nu >= 56 : nu > 64 && tiles <= 6ull * cus;
+}
+
+template <Op O>
+int launch_stream(const MvParams &p, const void *act, uint64_t tiles, const MatvecArgs &a) {
+    if constexpr (kind_of<O>() != kPTQ1) {
+        return -2;
+    } else {
+        hipLaunchKernelGGL(k_mv_stream_lut<O>, dim3(static_cast<uint32_t>(tiles < a.cus ? tiles : a.cus)),
+                           dim3(kLutThreads), stream_lds<O>(), a.stream, p, act);
+        return launch_status();
+    }
+}
+
 template <Op O>
 int launch_op(const MatvecArgs &a, const void *act, float *out) {
     const uint32_t nu = static_cast<uint32_t>(a.cols / unit_weights<O>());
@@ -2834,6 +3020,7 @@ int launch_op(const MatvecArgs &a, const void *act, float *out) {
         // Rows of up to 64 units from half a tile per CU (against the split kernel below one
         // tile per CU, the split-pair table kernel above): 10240x5120 10.0 -> 7.3, 12288x5120
         // 10.1 -> 7.6, 17408x5120 21.3 -> 10.6.
+        if (!quant && nmat == 1 && takes_stream<O>(tiles, nu, a.cus)) return launch_stream<O>(p, act, tiles, a);
         const uint32_t sgrid = static_cast<uint32_t>(tiles < a.cus ? tiles : a.cus);
         if (!quant && nmat == 1 && 2 * tiles > a.cus && nu <= 64) {
             if (const uint32_t lds = lut_spread_lds<O>(static_cast<uint32_t>(tiles), sgrid, nu)) {
@@ -2906,8 +3093,9 @@ int launch_op(const MatvecArgs &a, const void *act, float *out) {
         if (quant || nmat != 1) return -2;
         const uint32_t grid = static_cast<uint32_t>(tiles < a.cus ? tiles : a.cus);
         if constexpr (kind_of<O>() == kPTQ1) {
-            // The tile's units over 16 wavefronts with their terms in LDS when they fit beside
-            // the table, else one wavefront per tile.
+            // The tile's units over 16 wavefronts: with all their terms in LDS when they fit
+            // beside the table, else sixteen at a time, else one wavefront per tile.
+            if (O == Op::PTQ1_PINNED && nu <= kStreamMaxUnits) return launch_stream<O>(p, act, tiles, a);
             if (const uint32_t lds = lut_spread_lds<O>(static_cast<uint32_t>(tiles), grid, nu))
                 hipLaunchKernelGGL((k_mv_rows_lut<O, kLutSpread>), dim3(grid), dim3(kLutThreads), lds, a.stream, p, act);
             else
@@ -2965,6 +3153,7 @@ template <Op O>
 bool op_needs_prepared(const MatvecArgs &a) {
     const uint64_t tiles = (a.rows + kTile - 1) / kTile;
     if (!a.w2 && tiles >= a.cus) return true;
+    if (!a.w2 && a.act_fit && takes_stream<O>(tiles, static_cast<uint32_t>(a.cols / unit_weights<O>()), a.cus)) return true;
     SplitPlan pl;
     const uint32_t nu = static_cast<uint32_t>(a.cols / unit_weights<O>());
     return !plan_split<O>(a.rows, nu, static_cast<uint32_t>(a.cols), true, a.w2 ? 2u : 1u, a.cus, &pl,

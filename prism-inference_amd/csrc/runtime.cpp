@@ -56,11 +56,13 @@ int project_f32_dev(prism_hip_ctx *c, const Weight &w, const float *x, uint32_t 
     }
     if (w.tiled) {
         MatvecArgs a = f32_args(c, w, x, tokens, pinned, out, residual, s);
-        if (tokens > 1) {
-            const size_t act = act_bytes(contract_for(w.kind, w.cols, pinned), w.cols, tokens);
-            a.act_fit = act <= scratch_room(c, sc, role, act);
+        bool prepared = tiled_needs_prepared(a);
+        if (prepared) {
+            const size_t need = act_bytes(contract_for(w.kind, w.cols, pinned), w.cols, tokens);
+            a.act_fit = need <= scratch_room(c, sc, role, need);
+            if (!a.act_fit) prepared = tiled_needs_prepared(a);
         }
-        if (!tiled_needs_prepared(a)) return run_matvec(c, a, true, &scr);
+        if (!prepared) return run_matvec(c, a, true, &scr);
     }
     const int contract = contract_for(w.kind, w.cols, pinned);
     void *act = nullptr;
