@@ -2911,7 +2911,12 @@ struct SplitPlan {
 
 // Split-mode geometry: enough lane groups per row that the tiles cover every CU,
 // then enough wavefronts per workgroup for ~8 resident wavefronts per CU, never
-// more K-split ways than the row has units.
+// more K-split ways than the row has units.  Sixteen per CU on long rows from a quarter tile
+// per CU: each lane walks its units with one load ahead, so its walk is memory latency, and
+// more lanes shorten it.  Measured (one token, f32 or prepared input as the dispatch has it,
+// us, 8 / 16): 5120 x 17408 PQ2 15.4 / 13.5, Q2_K 13.1 / 11.5, Q8_0 25.0 / 21.6, TQ1_0 15.9 /
+// 14.1; PTQ1, whose decode bounds it, loses (17.1 / 18.2), and so does a Q2_K prologue (15.1 /
+// 16.3: its workgroups quantize longer than they read).
 // max_lpr caps the lane groups per row (a workgroup then owns at least 64/max_lpr rows).
 template <Op O>
 bool plan_split(uint64_t rows, uint32_t nu, uint32_t cols, bool quant, uint32_t nmat, uint32_t cus, SplitPlan *pl,
@@ -2919,8 +2924,11 @@ bool plan_split(uint64_t rows, uint32_t nu, uint32_t cols, bool quant, uint32_t 
     const uint64_t tiles = (rows + kTile - 1) / kTile;
     uint32_t lpr = 1;
     while (lpr < max_lpr && tiles * lpr < cus && lpr * 2 <= nu) lpr *= 2;
+    const bool wide = kind_of<O>() != kPTQ1 && !(quant && (O == Op::Q2K || O == Op::TQ2)) && nmat == 1 &&
+                      cols >= 10240 && 4 * tiles > cus;
+    const uint64_t waves = (wide ? 16ull : 8ull) * cus;
     uint32_t ks = 1;
-    while (ks * 2 * nmat <= kSplitMaxWaves && ks * 2 * lpr <= nu && tiles * lpr * ks * 2 * nmat <= 8ull * cus) ks *= 2;
+    while (ks * 2 * nmat <= kSplitMaxWaves && ks * 2 * lpr <= nu && tiles * lpr * ks * 2 * nmat <= waves) ks *= 2;
     // A quantizing prologue wants several wavefronts per workgroup: trade lane groups
     // for wavefronts while the workgroup has fewer than four.
     while (quant && ks * nmat < 4 && lpr > 1 && ks * 2 * nmat <= kSplitMaxWaves) {
@@ -2957,15 +2965,34 @@ bool plan_split(uint64_t rows, uint32_t nu, uint32_t cols, bool quant, uint32_t 
 // (20000 rows 9.8 / 11.7, 11.8 / 13.8) and past them whole tiles took 58.5 / 23.7, 96.4 / 37.3;
 // 40000 rows x 10240 60.4 / 33.1, about eight microseconds more per tile and CU.
 // Below half a tile per CU the split kernel is ahead (pinned 8000 x 10240 16.7 / 18.6, 2048 x
-// 17408 15.8 / 27.4) but for the longest pinned rows (4096 x 17408 29.9 / 27.3, 8000 x 17408
-// 39.5 / 27.8: every one of its workgroups stages the whole input).
+// 17408 15.8 / 27.4) but for the longest pinned rows (4096 x 17408 29.9 / 27.3, 8000 x 14336
+// 32.6 / 24, 8000 x 17408 39.5 / 27.8: every one of its workgroups stages the whole input).
 template <Op O>
 bool takes_stream(uint64_t tiles, uint32_t nu, uint32_t cus) {
     if constexpr (kind_of<O>() != kPTQ1) return false;
     if (nu > kStreamMaxUnits) return false;
-    if (2 * tiles <= cus) return O == Op::PTQ1_PINNED && nu >= 128 && 6 * tiles > cus;
+    if (2 * tiles <= cus) return O == Op::PTQ1_PINNED && nu >= 100 && 6 * tiles > cus;
     if constexpr (O == Op::PTQ1_PINNED) return tiles <= 4ull * cus && nu >= (tiles > 2ull * cus ? 16u : 25u);
     return tiles < cus ? nu >= 56 : nu > 64 && tiles <= 6ull * cus;
+}
+
+// Whether f32 input of one token on fewer tiles than CUs is quantized by a launch of its own
+// although the split kernel's prologue could: on long rows every one of its several hundred
+// workgroups quantizes the whole input.  Measured (us, prologue / separate quantizer, with the
+// wavefronts of plan_split): 5120 x 17408 PQ2 14.5 / 13.5, Q2_K 15.1 / 11.5, TQ1_0 16.2 / 14.1,
+// PTQ1 18.5 / 17.1, Q8_0 equal; 8000 x 10240 PQ2 11.2 / 10.8, Q2_K 10.7 / 9.8, TQ1_0 11.8 / 11.2;
+// above half a tile per CU, where prepared blocks run on the row-tile kernels, 12288 x 17408 PQ2
+// 21.2 / 20.5, Q2_K 21.8 / 20.0, Q8_0 40.1 / 37.2 but 12288 x 10240 PQ2 14.5 / 15.8, and PTQ1
+// rows of 36 to 55 units (12288 x 5120 10.8 / 9.2, 2048 inputs 5.4 / 7.6).  Fewer tiles gain
+// nothing (4096 x 10240 PQ2 7.8 / 8.9).
+template <Op O>
+bool long_rows_prepared(uint64_t tiles, uint64_t cols, uint32_t cus) {
+    if (4 * tiles <= cus || tiles >= cus || O == Op::PTQ1_PINNED) return false;
+    const bool few = 2 * tiles <= cus;
+    if constexpr (kind_of<O>() == kPTQ1) return few ? cols >= 14336 : cols >= 36 * 128 && cols < 56 * 128;
+    if constexpr (O == Op::Q8_0) return !few && cols >= 16384;
+    if constexpr (O == Op::TQ1) return few && cols >= 10240;
+    return cols >= (few ? 10240 : 16384);
 }
 
 template <Op O>
@@ -3153,7 +3180,10 @@ template <Op O>
 bool op_needs_prepared(const MatvecArgs &a) {
     const uint64_t tiles = (a.rows + kTile - 1) / kTile;
     if (!a.w2 && tiles >= a.cus) return true;
-    if (!a.w2 && a.act_fit && takes_stream<O>(tiles, static_cast<uint32_t>(a.cols / unit_weights<O>()), a.cus)) return true;
+    if (!a.w2 && a.act_fit &&
+        (takes_stream<O>(tiles, static_cast<uint32_t>(a.cols / unit_weights<O>()), a.cus) ||
+         long_rows_prepared<O>(tiles, a.cols, a.cus)))
+        return true;
     SplitPlan pl;
     const uint32_t nu = static_cast<uint32_t>(a.cols / unit_weights<O>());
     return !plan_split<O>(a.rows, nu, static_cast<uint32_t>(a.cols), true, a.w2 ? 2u : 1u, a.cus, &pl,

@@ -82,3 +82,21 @@ def test_gpu_pinned_gate_up_fold_matches_oracle(ctx, hidden, ffn):
     ctx.release(wg)
     ctx.release(wu)
     assert np.array_equal(np.asarray(got, np.float32).view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,pinned", [(ph.KIND_PQ2, True), (ph.KIND_PQ2, False), (ph.KIND_Q2_K, False), (ph.KIND_Q8_0, True),
+                                         (ph.KIND_TQ1_0, False), (ph.KIND_TQ2_0, False), (ph.KIND_PTQ1, False)])
+@pytest.mark.parametrize("per_cu4,extra,cols", [(1, 5, 10240), (1, 64, 17408), (2, 70, 16640), (2, 70, 4864)])
+def test_gpu_long_rows_separate_quantizer_matches_oracle(ctx, kind, pinned, per_cu4, extra, cols):
+    """A quarter to one tile per CU on long rows: sixteen split wavefronts per CU, and f32 input
+    quantized by a launch of its own."""
+    import oracle
+
+    rows = cu_count() * 16 * per_cu4 + extra
+    w = synth.weights(kind, rows, cols, seed=cols)
+    x = synth.activations(cols, seed=rows)
+    wid = ctx.weight(kind, cols, rows, w)
+    ref = oracle.matvec(kind, cols, rows, w, x, pinned, threads=THREADS)
+    got = ctx.project_f32(wid, rows, x, pinned=pinned)
+    ctx.release(wid)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
