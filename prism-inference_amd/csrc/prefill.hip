@@ -45,6 +45,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr uint32_t kRowsPerWg = 128, kTokAlign = 128;
+constexpr uint32_t kPinnedTokens = 64;  // tokens per workgroup of the pinned GEMM
 
 constexpr uint32_t sel_bytes(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
     return b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
@@ -221,6 +222,16 @@ struct PairDecoder {
     }
 };
 
+// Outer product of the rows' and the tokens' binary16 scales (bits in half 0 of the wavefront,
+// zero in half 1), in the MFMA output layout: each product has at most 22 significant bits, so
+// binary32 holds it exactly.  On the f16 matrix cores, which work beside the VALU; binary32
+// products (v_mfma_f32_32x32x2_f32) run on the VALU's own multipliers (measured, 8000 products
+// and 64000 FMAs per SIMD: f32 226 and 129 us apart, 355 together; f16 121 and 144, 163).
+__device__ __forceinline__ v16f scale_products(uint32_t row_bits, uint32_t token_bits) {
+    return __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, u32x2{row_bits, 0u}),
+                                                __builtin_bit_cast(v4h, u32x2{token_bits, 0u}), v16f{}, 0, 0, 0);
+}
+
 // s_waitcnt through the builtin (gfx9 encoding, other counters left at their maxima),
 // so the compiler's own wait bookkeeping sees it: vmcnt(0) / lgkmcnt(0).
 __device__ __forceinline__ void wait_vmcnt0() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -230,6 +241,13 @@ __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xC
 __device__ __forceinline__ void lds_barrier() {
     wait_lgkmcnt0();
     __builtin_amdgcn_s_barrier();
+}
+
+// 16 bytes to LDS, past the compiler's own bookkeeping: before an ordinary LDS store it waits
+// for every direct-to-LDS load in flight, whatever they write.  The next lds_barrier waits for it.
+__device__ __forceinline__ void lds_store16(u32x4 *p, u32x4 v) {
+    const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4 *)p));
+    asm volatile("ds_write_b128 %0, %1" ::"v"(at), "v"(v) : "memory");
 }
 
 template <int CT>
@@ -308,12 +326,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CT == 4 ? 2
     auto block = [&](uint32_t u, const uint8_t (&act)[8][2][kRun], const float4 (&scl)[NT],
                      uint8_t (&act_next)[8][2][kRun], float4 (&scl_next)[NT]) {
         uint32_t aw[4][4][2];  // [g][i][j]: pair h of quad 4j + i of group g
-        float dw = 0.0f;       // the lane's row scale in half 0, zero in half 1
+        uint32_t dw = 0;       // the lane's row scale (binary16 bits; CT > 1: binary32) in half 0, zero in half 1
         if (active) {
             PairDecoder dec(w, h);
 #pragma unroll
             for (int g = 0; g < 4; ++g) dec.group(g, aw[g]);
-            dw = h ? 0.0f : h2f(w.tl >> 16);
+            dw = h ? 0u : CT == 1 ? w.tl >> 16 : __float_as_uint(h2f(w.tl >> 16));
         }
         // The next block streams in while this one is multiplied.
         if (u + 1 < nu) {
@@ -322,8 +340,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CT == 4 ? 2
         }
         if (active) {
             // The scales d_w of the lane's 16 output rows, in the MFMA output layout: the
-            // outer product of the rows' scales with ones (exact).
-            const v16f d = __builtin_amdgcn_mfma_f32_32x32x2f32(dw, h ? 0.0f : 1.0f, v16f{}, 0, 0, 0);
+            // outer product of the rows' scales with ones.
+            // (More than 32 tokens sit at the register limit, where the f16 form spilled:
+            // 6144 x 2048, 2048 tokens 101.7 -> 104.5 us; 32 tokens 12288 x 4096, 500 tokens
+            // 114.9 -> 108.1.)
+            v16f d;
+            if constexpr (CT == 1)
+                d = scale_products(dw, h ? 0u : 0x3c00u);
+            else
+                d = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(dw), h ? 0.0f : 1.0f, v16f{}, 0, 0, 0);
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 const float4 sg4 = scl[32 * ct + r32];
@@ -456,19 +481,19 @@ __global__ __launch_bounds__(64 * 4 * kPhases) void k_prefill_ptq1_split(const u
         const uint32_t u = kPhases * r + phase, un = u + kPhases;
         const bool mine = u < nu && active;
         uint32_t aw[4][4][2];
-        float dw = 0.0f;
+        uint32_t dw = 0;
         if (mine) {
             PairDecoder dec(w, h);
 #pragma unroll
             for (int g = 0; g < 4; ++g) dec.group(g, aw[g]);
-            dw = h ? 0.0f : h2f(w.tl >> 16);
+            dw = h ? 0u : w.tl >> 16;
         }
         if (un < nu) {
             stage(un, act_next, scl_next);
             if (active) load_block_codes(rw_, un * trp * 28u, trp, row, w);
         }
         if (mine) {
-            const v16f d = __builtin_amdgcn_mfma_f32_32x32x2f32(dw, h ? 0.0f : 1.0f, v16f{}, 0, 0, 0);
+            const v16f d = scale_products(dw, h ? 0u : 0x3c00u);
             const float4 sg4 = scl[phase][r32];
             const float sg[4] = {sg4.x, sg4.y, sg4.z, sg4.w};
             v16f tt;
@@ -529,57 +554,124 @@ __global__ __launch_bounds__(64 * 4 * kPhases) void k_prefill_ptq1_split(const u
     if (bad) raise_error(err, kErrNonfinite);
 }
 
-// The pinned contract (dot_q8_groups_pinned, src/kernels.rs:1102-1147) on the same
-// tiles: per (token, row) four binary32 lanes L[l] = fma(I_l, dd_g, L[l]) with
-// dd_g = fl(d_w * A_g.scale), group by group, and (L0 + L1) + (L2 + L3) at the end.  In
-// the pinned operand order one v_mfma_f32_32x32x8_f16 per (group, native lane) sums
-// exactly that lane's eight elements, half h of the wavefront supplying four of them
-// (binary16-exact operands, |I| <= 8*127): four MFMAs per group, each as long as one
-// K=16 MFMA on gfx950, and no masking.  20 VALU per output and block instead of 6 (the
-// four dd_g and sixteen FMAs): 32 tokens per workgroup keep the 64 lane accumulators of
-// a wavefront in registers.
+// Half of PairDecoder's work for the pinned order: half j of the block's native lanes, l = j and
+// j + 2.  Their quads (pair_base) come from code dwords A_j and A_{j+2}, B_j and tail quad j
+// (120, 124): groups 0 and 1 take two digits of each A dword, group 2 the last one and B's first
+// two, group 3 B's other three and the tail.  Every dword is so decoded by one half only.
+struct LaneDecoder {
+    uint32_t la0, la1, lb, tb;
+
+    __device__ __forceinline__ void start(const uint32_t (&raw)[4], uint32_t h) {
+        const uint32_t sel = h ? sel_bytes(1, 12, 3, 12) : sel_bytes(0, 12, 2, 12);  // bytes h, h+2
+        la0 = perm(raw[0], raw[0], sel);
+        la1 = perm(raw[1], raw[1], sel);
+        lb = perm(raw[2], raw[2], sel);
+        tb = perm(raw[3], raw[3], h ? sel_bytes(1, 12, 1, 12) : sel_bytes(0, 12, 0, 12));
+    }
+    // Operands of native lanes j (a0) and j + 2 (a1) of group g; tail = the tail's multipliers.
+    __device__ __forceinline__ void group(int g, uint32_t tail, u32x2 &a0, u32x2 &a1) {
+        if (g < 2) {
+            a0.x = PairDecoder::next(la0);
+            a0.y = PairDecoder::next(la0);
+            a1.x = PairDecoder::next(la1);
+            a1.y = PairDecoder::next(la1);
+        } else if (g == 2) {
+            a0.x = PairDecoder::next(la0);
+            a1.x = PairDecoder::next(la1);
+            a0.y = PairDecoder::next(lb);
+            a1.y = PairDecoder::next(lb);
+        } else {
+            a0.x = PairDecoder::next(lb);
+            a1.x = PairDecoder::next(lb);
+            a0.y = PairDecoder::next(lb);
+            a1.y = f16_pair((pair_mul(tb, tail) & 0x00ff00ffu) * 3u);
+        }
+    }
+};
+
+// The pinned contract (dot_q8_groups_pinned, src/kernels.rs:1102-1147): per (token, row) four
+// binary32 lanes L[l] = fma(I_l, dd_g, L[l]) with dd_g = fl(d_w * A_g.scale), group by group,
+// and (L0 + L1) + (L2 + L3) at the end.  In the pinned operand order one
+// v_mfma_f32_32x32x8_f16 per (group, native lane) sums exactly that lane's eight elements, half
+// h of the wavefront supplying four of them (binary16-exact operands, |I| <= 8*127): four MFMAs
+// per group, each as long as one K=16 MFMA on gfx950, and no masking.  20 VALU per output and
+// block instead of 6 (the four dd_g, on the matrix pipe, and sixteen FMAs).
+//
+// The VALU bounds it (256 FMAs per 32 x 32 outputs and block, 1024 cycles, and about 200 more
+// instructions when every wavefront decoded its own 32 rows for 32 tokens).  So the four
+// wavefronts of a workgroup are two of rows by two of tokens on one 64-row tile and 64 tokens:
+// the two that share 32 rows decode half of them each (LaneDecoder) into LDS.  A block runs in
+// two halves of two groups, each half of the codes and of the operands in its own LDS buffer:
+// while one half is multiplied, the next half's codes stream into the other and its operands
+// are decoded into it, and one barrier a half hands both over (34 KiB, four workgroups a CU).
+template <bool HALF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_prefill_ptq1_pinned(
     const uint8_t *__restrict__ W, uint32_t rows, uint32_t nu, const _Float16 *__restrict__ xh,
     const float *__restrict__ sc, uint32_t M, uint32_t Mp, uint32_t xcd_major, float *__restrict__ out,
     int *__restrict__ err) {
-    constexpr uint32_t NT = 32;
+    constexpr uint32_t NT = kPinnedTokens;
     constexpr uint32_t kRun = NT * 8;  // bytes of one (g, l, h) run of one block
-    __shared__ __attribute__((aligned(16))) uint8_t act0[32][kRun];
-    __shared__ __attribute__((aligned(16))) uint8_t act1[32][kRun];
+    // Half 0: groups 0 and 1; half 1: groups 2 and 3.  act[4 (g % 2) + l][h][token][8 bytes],
+    // opa[row half][g % 2][j][h][row][16 bytes] (native lanes j and j + 2), scl[token] by block parity.
+    __shared__ __attribute__((aligned(16))) uint8_t act0[16][kRun];
+    __shared__ __attribute__((aligned(16))) uint8_t act1[16][kRun];
+    __shared__ __attribute__((aligned(16))) uint8_t act2[16][kRun];
+    __shared__ __attribute__((aligned(16))) uint8_t act3[16][kRun];
+    __shared__ __attribute__((aligned(16))) u32x4 opa0[2][2][2][2][32];
+    __shared__ __attribute__((aligned(16))) u32x4 opa1[2][2][2][2][32];
     __shared__ __attribute__((aligned(16))) float4 scl0[NT];
     __shared__ __attribute__((aligned(16))) float4 scl1[NT];
     const uint32_t lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t bx = xcd_major ? blockIdx.y : blockIdx.x;
+    const uint32_t hw = wave >> 1, tw = wave & 1;  // row half, token half
+    const uint32_t tile = xcd_major ? blockIdx.y : blockIdx.x;
     const uint32_t by = xcd_major ? blockIdx.x + 8 * blockIdx.z : blockIdx.y;
-    const uint32_t tile = 2 * bx + (wave >> 1), hw = wave & 1;
-    const uint32_t tiles = (rows + kTile - 1) / kTile;
-    const uint32_t t0 = by * NT;
-    const uint32_t row_bytes = nu * 28;
-    uint32_t trows = 0;
-    if (tile < tiles) {
-        const uint32_t left = rows - tile * kTile;
-        trows = left < kTile ? left : kTile;
-    }
-    const bool active = 32 * hw < trows;  // uniform per wavefront
-    const uint32_t trp = (trows + 7u) & ~7u;
+    const uint32_t t0 = by * NT, row_bytes = nu * 28;
+    const uint32_t left = rows - tile * kTile;  // tile * kTile < rows
+    const uint32_t trows = left < kTile ? left : kTile, trp = (trows + 7u) & ~7u;
+    // Uniform per wavefront: rows and tokens of its quarter exist.  The others still decode and
+    // stage (their padding rows read zeros or other bytes of the tile, and are never stored).
+    const bool active = 32 * hw < trows && t0 + 32 * tw < M;
     const __amdgpu_buffer_rsrc_t rw =
-        make_rsrc(W + static_cast<size_t>(active ? tile : 0) * kTile * row_bytes, active ? trp * row_bytes : 0u);
+        make_rsrc(W + static_cast<size_t>(tile) * kTile * row_bytes, trp * row_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(xh, nu * 8u * Mp * 32u);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(sc, nu * Mp * 16u);
     const uint32_t row = 32 * hw + r32, out0 = 32 * hw + 4 * h;  // tile rows
 
-    // Block u's codes (32 runs of NT*8 bytes, each contiguous in xh and in LDS; one
-    // instruction moves four runs, lane l tokens 2(l%16), 2(l%16)+1 of run l/16) and the
-    // scales of the workgroup's tokens.
-    auto stage = [&](uint32_t u, uint8_t (&act)[32][kRun], float4 (&scl)[NT]) {
-        for (uint32_t i = wave; i < 8; i += 4)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void *)(&act[4 * i][0]), 16,
-                                                     ((u * 32 + 4 * i + lane / 16) * Mp + t0 + 2 * (lane % 16)) * 8u, 0,
-                                                     0, 0);
-        if (wave == 0 && lane < NT)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(&scl[0]), 16, (u * Mp + t0 + lane) * 16u, 0,
-                                                     0, 0);
+    // Half `half` of block u's codes: 16 runs of NT * 8 bytes, each contiguous in xh and in LDS;
+    // one instruction moves two runs, lane l tokens 2 (l % 32), + 1 of run l / 32.
+    auto stage = [&](uint32_t u, uint32_t half, uint8_t (&act)[16][kRun]) {
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            const uint32_t k = 2 * (wave + 4 * i);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rx, (lds_void *)(&act[k][0]), 16,
+                ((u * 32 + 16 * half + k + lane / 32) * Mp + t0 + 2 * (lane % 32)) * 8u, 0, 0, 0);
+        }
+    };
+    auto stage_scales = [&](uint32_t u, float4 (&scl)[NT]) {
+        if (lane < NT / 4)  // every wavefront a quarter: all issue the same loads
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(&scl[wave * (NT / 4)]), 16,
+                                                     (u * Mp + t0 + wave * (NT / 4) + lane) * 16u, 0, 0, 0);
+    };
+    // The dwords of LaneDecoder's half tw of the lane's row: A_tw, A_{tw+2}, B_tw and the tail.
+    uint32_t raw[4];
+    auto load = [&](uint32_t u) {
+        const uint32_t seg = u * trp * 28u;
+        raw[0] = bload1(rw, seg + 16u * row + 4u * tw);
+        raw[1] = bload1(rw, seg + 16u * row + 4u * tw + 8u);
+        raw[2] = bload1(rw, seg + 16u * trp + 8u * row + 4u * tw);
+        raw[3] = bload1(rw, seg + 24u * trp + 4u * row);
+    };
+    LaneDecoder dec;
+    const uint32_t tail = tw ? (9u | (27u << 16)) : (1u | (3u << 16));
+    auto decode = [&](int g0, u32x4 (&opa)[2][2][2][2][32]) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            u32x2 a0, a1;
+            dec.group(g0 + g, tail, a0, a1);
+            lds_store16(&opa[hw][g][tw][h][r32], u32x4{a0.x, a0.y, a1.x, a1.y});
+        }
     };
 
     float L[4][16];
@@ -588,52 +680,88 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 #pragma unroll
         for (int r = 0; r < 16; ++r) L[l][r] = 0.0f;
     const v16f zero = {};
-
-    RawBlock w = {};  // stays zero in an inactive wavefront
-    stage(0, act0, scl0);
-    if (active) load_block_codes(rw, 0, trp, row, w);
-    wait_vmcnt0();
-    lds_barrier();
-    auto block = [&](uint32_t u, const uint8_t (&act)[32][kRun], const float4 (&scl)[NT],
-                     uint8_t (&act_next)[32][kRun], float4 (&scl_next)[NT]) {
-        PairDecoder dec(w, h);
-        const float dw = h ? 0.0f : h2f(w.tl >> 16);  // the lane's row scale in half 0, zero in half 1
-        if (u + 1 < nu) {
-            stage(u + 1, act_next, scl_next);
-            if (active) load_block_codes(rw, (u + 1) * trp * 28u, trp, row, w);
-        }
-        if (active) {
-            const float4 sg4 = scl[r32];
-            const float sg[4] = {sg4.x, sg4.y, sg4.z, sg4.w};
+    // Two groups of a block from (act, opa): da is the lane's row scale (binary16 bits) in lanes
+    // 0..31, else 0.
+    auto multiply = [&](uint32_t da, const float (&sg)[2], const uint8_t (&act)[16][kRun],
+                        const u32x4 (&opa)[2][2][2][2][32]) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                // dd[r] = fl(d_w * A_g.scale) for every (row, token) of the tile, as the
-                // outer product of the rows' and tokens' scales on the matrix pipe: K = 2
-                // with the second term zero, one rounding (no product is subnormal: both
-                // scales are binary16 values).
-                const v16f dd = __builtin_amdgcn_mfma_f32_32x32x2f32(dw, h ? 0.0f : sg[g], zero, 0, 0, 0);
-                uint32_t aw[4][2];
-                dec.group(g, aw);
+        for (int g = 0; g < 2; ++g) {
+            // dd[r] = fl(d_w * A_g.scale) for every (row, token) of the tile, as an outer
+            // product: HALF where this library's quantizer made the scales, which are binary16
+            // values then; a caller's own blocks may hold any binary32 scale (K = 2 with the
+            // second term zero, one rounding).
+            v16f dd;
+            if constexpr (HALF)
+                dd = scale_products(da, h ? 0u : __builtin_bit_cast(uint16_t, static_cast<_Float16>(sg[g])));
+            else
+                dd = __builtin_amdgcn_mfma_f32_32x32x2f32(h2f(da), h ? 0.0f : sg[g], zero, 0, 0, 0);
 #pragma unroll
-                for (int l = 0; l < 4; ++l) {
-                    const v4h b = *reinterpret_cast<const v4h *>(&act[(4 * g + l) * 2 + h][r32 * 8]);
-                    const u32x2 a = {aw[l][0], aw[l][1]};
-                    const v16f i = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, a), b, zero, 0, 0, 0);
+            for (int j = 0; j < 2; ++j) {
+                const u32x4 a2 = opa[hw][g][j][h][r32];  // native lanes j and j + 2
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int l = j + 2 * k;
+                    const v4h b = *reinterpret_cast<const v4h *>(&act[(4 * g + l) * 2 + h][(32 * tw + r32) * 8]);
+                    const v4h a = __builtin_bit_cast(v4h, u32x2{a2[2 * k], a2[2 * k + 1]});
+                    const v16f i = __builtin_amdgcn_mfma_f32_32x32x8f16(a, b, zero, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 16; ++r) L[l][r] = __builtin_fmaf(i[r], dd[r], L[l][r]);
                 }
             }
         }
-        wait_vmcnt0();
+    };
+
+    // Half n = 2u + half is staged three halves ahead, into buffer n % 4.  Each wavefront issues,
+    // in this order, 2 loads in a first half (codes of half n + 3) and 7 in a second (2 of codes,
+    // 1 of scales, 4 of weights), also past the row's end (the buffers' bounds then yield zeros),
+    // so the loads still allowed in flight when half n + 1 must have landed are those counts.
+    load(0);
+    stage(0, 0, act0);
+    stage_scales(0, scl0);
+    stage(0, 1, act1);
+    uint32_t dw = h ? 0u : raw[3] >> 16;
+    dec.start(raw, h);
+    stage(1, 0, act2);
+    stage_scales(1, scl1);
+    load(1);
+    decode(0, opa0);
+    wait_vmcnt0();
+    lds_barrier();
+    auto block = [&](uint32_t u, const uint8_t (&a0)[16][kRun], const uint8_t (&a1)[16][kRun],
+                     uint8_t (&n0)[16][kRun], uint8_t (&n1)[16][kRun], float4 (&scl)[NT]) {
+        // First half, while the second half's operands are made.
+        stage(u + 1, 1, n1);
+        decode(2, opa1);
+        float4 sg = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (active) {
+            sg = scl[32 * tw + r32];
+            const float s01[2] = {sg.x, sg.y};
+            multiply(dw, s01, a0, opa0);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F79);  // vmcnt(9): half 2u + 1 has landed
+        lds_barrier();
+        // Second half, while the next block's first operands are made.
+        const uint32_t d1 = dw;
+        stage(u + 2, 0, n0);
+        stage_scales(u + 2, scl);
+        dw = h ? 0u : raw[3] >> 16;
+        dec.start(raw, h);
+        load(u + 2);
+        decode(0, opa0);
+        if (active) {
+            const float s23[2] = {sg.z, sg.w};
+            multiply(d1, s23, a1, opa1);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F7D);  // vmcnt(13): half 2u + 2 and its scales have landed
         lds_barrier();
     };
     for (uint32_t u = 0; u < nu; u += 2) {
-        block(u, act0, scl0, act1, scl1);
-        if (u + 1 < nu) block(u + 1, act1, scl1, act0, scl0);
+        block(u, act0, act1, act0, act3, scl0);
+        if (u + 1 < nu) block(u + 1, act2, act3, act2, act1, scl1);
     }
-    if (!active) return;
-    const uint32_t t = t0 + r32;
-    if (t >= M) return;
+    wait_vmcnt0();  // loads past the row's end still write LDS
+    const uint32_t t = t0 + 32 * tw + r32;
+    if (!active || t >= M) return;
     bool bad = false;
     float *yr = out + static_cast<size_t>(t) * rows + static_cast<size_t>(tile) * kTile;
 #pragma unroll
@@ -720,10 +848,11 @@ static int launch_ptq1(const void *w_tiled, uint64_t cols, uint64_t rows, const 
     const auto W = static_cast<const uint8_t *>(w_tiled);
     const uint32_t R = static_cast<uint32_t>(rows), nu = K / 128;
     if (pinned) {
-        const uint32_t groups = (M + 31) / 32;  // token groups holding real tokens
-        const uint32_t xcd_major = groups % 8 == 0 && gx <= 65535;
-        const dim3 grid = xcd_major ? dim3(8, gx, groups / 8) : dim3(gx, groups);
-        hipLaunchKernelGGL(k_prefill_ptq1_pinned, grid, dim3(256), 0, s, W, R, nu, xh, sc, M, Mp, xcd_major, out, err);
+        const uint32_t groups = (M + kPinnedTokens - 1) / kPinnedTokens;  // token groups holding real tokens
+        const uint32_t tiles = static_cast<uint32_t>((rows + kTile - 1) / kTile);
+        const uint32_t xcd_major = groups % 8 == 0 && tiles <= 65535;
+        const dim3 grid = xcd_major ? dim3(8, tiles, groups / 8) : dim3(tiles, groups);
+        hipLaunchKernelGGL(k_prefill_ptq1_pinned<!BLOCKS>, grid, dim3(256), 0, s, W, R, nu, xh, sc, M, Mp, xcd_major, out, err);
         return launch_status();
     }
     // Tokens per workgroup (measured, 6144 x 2048): 64 keeps three wavefronts per SIMD

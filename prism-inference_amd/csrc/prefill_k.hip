@@ -56,6 +56,7 @@ namespace prism {
 
 namespace {
 
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -312,8 +313,11 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
 }
 
-// FUSED (PQ2 only): dot_pq2<true>'s fma(d, s, o) instead of o + d * s.
-template <uint32_t KIND, int CT, bool FUSED>
+// ALT, PQ2: dot_pq2<true>'s fma(d, s, o) instead of o + d * s.  ALT, Q8_0: the tokens' scales are
+// binary16 values (this library's quantizer made them, not the caller), so a block's scale
+// products are exact on the f16 matrix cores, beside the VALU; binary32 products there take the
+// VALU's own multipliers (prefill.hip, scale_products).
+template <uint32_t KIND, int CT, bool ALT>
 __global__ __launch_bounds__(256) void k_prefill_kq(const uint8_t *__restrict__ W, uint32_t rows, uint32_t nu,
                                                     const uint8_t *__restrict__ xq, const float *__restrict__ as,
                                                     const _Float16 *__restrict__ bs, uint32_t M, uint32_t Mp,
@@ -545,15 +549,20 @@ __global__ __launch_bounds__(256) void k_prefill_kq(const uint8_t *__restrict__ 
                 // I_s one K-step.
 #pragma unroll
                 for (int s = 0; s < 8; ++s) {
-                    const float ws = h ? 0.0f : h2f((wsc[s >> 2][(s >> 1) & 1] >> (16 * (s & 1))) & 0xffffu);
+                    const uint32_t wb = h ? 0u : (wsc[s >> 2][(s >> 1) & 1] >> (16 * (s & 1))) & 0xffffu;
 #pragma unroll
                     for (int ct = 0; ct < CT; ++ct) {
                         // Read by every lane: a branch around the read (lanes of half 1 need
                         // none) lets the compiler sink the chain below all eight blocks' MFMAs,
                         // whose results then fill the registers.
                         const float sa = scl[s][32 * ct + r32];
-                        const float a = h ? 0.0f : sa;
-                        const v16f dd = __builtin_amdgcn_mfma_f32_32x32x2f32(ws, a, v16f{}, 0, 0, 0);
+                        v16f dd;  // fl(ws_s * as_s)
+                        if constexpr (ALT)
+                            dd = __builtin_amdgcn_mfma_f32_32x32x8f16(
+                                __builtin_bit_cast(v4h, u32x2{wb, 0u}),
+                                v4h{static_cast<_Float16>(h ? 0.0f : sa), 0, 0, 0}, v16f{}, 0, 0, 0);
+                        else
+                            dd = __builtin_amdgcn_mfma_f32_32x32x2f32(h2f(wb), h ? 0.0f : sa, v16f{}, 0, 0, 0);
                         const v16i is = kstep(s, ct, v16i{});
 #pragma unroll
                         for (int r = 0; r < 16; ++r) o[ct][r] = o[ct][r] + dd[r] * static_cast<float>(is[r]);
@@ -583,7 +592,7 @@ __global__ __launch_bounds__(256) void k_prefill_kq(const uint8_t *__restrict__ 
 #pragma unroll
                         for (int r = 0; r < 16; ++r) {
                             const float sv = static_cast<float>(ib[ct][b][r]);
-                            o[ct][r] = FUSED ? __builtin_fmaf(dd[r], sv, o[ct][r]) : o[ct][r] + dd[r] * sv;
+                            o[ct][r] = ALT ? __builtin_fmaf(dd[r], sv, o[ct][r]) : o[ct][r] + dd[r] * sv;
                         }
                     }
                 }
@@ -706,7 +715,7 @@ static int launch_k(uint32_t kind, const void *w_tiled, uint64_t cols, uint64_t 
     else if (kind == kTQ2_0)
         nt == 64 ? go(k_prefill_kq<kTQ2_0, 2, false>) : go(k_prefill_kq<kTQ2_0, 1, false>);
     else if (kind == kQ8_0)
-        go(k_prefill_kq<kQ8_0, 1, false>);
+        go(k_prefill_kq<kQ8_0, 1, !BLOCKS>);
     else if (pinned)
         nt == 64 ? go(k_prefill_kq<kPQ2, 2, true>) : go(k_prefill_kq<kPQ2, 1, true>);
     else
