@@ -18,15 +18,21 @@
 
 namespace prism {
 
+// Column i of the token rows blockIdx.y, + gridDim.y, ...: a flat index took a 64-bit remainder
+// per element (333 x 6144: 6.5 us of 24 MB).
 __global__ __launch_bounds__(256) void k_swiglu(const float *__restrict__ g, const float *__restrict__ u,
-                                                float *__restrict__ h, uint64_t n, uint64_t total, int pinned,
+                                                float *__restrict__ h, uint64_t n, uint32_t tokens, int pinned,
                                                 int *__restrict__ err) {
-    const uint64_t idx = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const uint64_t i = idx % n;
-    const float r = swiglu_one(g[idx], u[idx], i, n, pinned);
-    h[idx] = r;
-    if (!finite(r)) raise_error(err, kErrNonfinite);
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    bool bad = false;
+    for (uint32_t t = blockIdx.y; t < tokens; t += gridDim.y) {
+        const uint64_t at = t * n + i;
+        const float r = swiglu_one(g[at], u[at], i, n, pinned);
+        h[at] = r;
+        bad |= !finite(r);
+    }
+    if (bad) raise_error(err, kErrNonfinite);
 }
 
 __global__ __launch_bounds__(256) void k_add_residual(float *__restrict__ out, const float *__restrict__ res,
@@ -149,10 +155,9 @@ __global__ void k_fill_i32(int *p, int v, uint32_t n) {
 
 int launch_swiglu(const float *gate, const float *up, float *h, uint64_t n, uint32_t tokens, int pinned, int *err,
                   hipStream_t s) {
-    const uint64_t total = n * tokens;
-    if (total == 0) return 0;
-    hipLaunchKernelGGL(k_swiglu, dim3(static_cast<uint32_t>((total + 255) / 256)), dim3(256), 0, s, gate, up, h, n,
-                       total, pinned, err);
+    if (n == 0 || tokens == 0) return 0;
+    hipLaunchKernelGGL(k_swiglu, dim3(static_cast<uint32_t>((n + 255) / 256), tokens < 65535 ? tokens : 65535), dim3(256),
+                       0, s, gate, up, h, n, tokens, pinned, err);
     return launch_status();
 }
 

@@ -9,6 +9,7 @@
 #include "runtime_internal.hpp"
 
 #include <cmath>
+#include <functional>
 
 using namespace prism;
 using namespace prism::rt;
@@ -148,9 +149,8 @@ int prepare_weight(prism_hip_ctx *c, prism_weight_id wid, int path, const Weight
 }
 
 int finish(prism_hip_ctx *c, float *host_out, const float *dev_out, size_t n) {
-    hipError_t e = hipMemcpyAsync(host_out, dev_out, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream);
-    if (e != hipSuccess) return hip_fail(c, e, "copy output");
-    return drain(c, c->stream);
+    const int rc = download(c, host_out, dev_out, sizeof(float) * n, c->stream, "copy output");
+    return rc ? rc : drain(c, c->stream);
 }
 
 // The Hadamard block of a rotated down projection (project_f32_ffn_chain's
@@ -283,9 +283,11 @@ int group_tokens_impl(prism_hip_ctx *c, const Weight *const *w, uint32_t n, cons
 // (multi-token kernels read each weight once per batch), one SwiGLU launch, and down
 // over all tokens.  Every token row is its own single-token chain's result.  h, if not
 // NULL, receives the SwiGLU rows; without a down projection `out` is that vector.
+// residual_upload, if any (more than one token), is called before the first launch that reads
+// `residual`.
 int ffn_tokens_impl(prism_hip_ctx *c, const Weight &g, const Weight &u, const Weight *d, const float *x,
                     const float *residual, uint32_t tokens, int pinned, float *out, float *h, hipStream_t s,
-                    uint32_t hb = 0) {
+                    uint32_t hb = 0, const std::function<int()> &residual_upload = nullptr) {
     const prism_tensor_desc dd = d ? desc_of(*d) : prism_tensor_desc{};
     if (!ffn_eligible(desc_of(g), desc_of(u), d ? &dd : nullptr))
         return fail(c, PRISM_ERR_UNSUPPORTED, "FFN chain needs gate/up [ffn][hidden] and down [hidden][ffn] of one packed kind");
@@ -307,6 +309,8 @@ int ffn_tokens_impl(prism_hip_ctx *c, const Weight &g, const Weight &u, const We
     if (!rc)
         rc = launch_result(c, launch_swiglu(gu_out[0], gu_out[1], hv, g.rows, tokens, pinned, c->err, s),
                            "swiglu launch");
+    // Gate, up and SwiGLU are queued: the residual can cross beside them.
+    if (!rc && residual_upload) rc = residual_upload();
     if (rc || !d) return rc;
     const float *din = nullptr;
     rc = down_input(c, hv, g.rows, tokens, hb, s, &din);
@@ -351,6 +355,8 @@ void prism_hip_destroy(prism_hip_ctx *c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     prism_hip_weight_release_all(c);
+    if (c->staging.side) (void)hipStreamSynchronize(c->staging.side);
+    staging_free(c->staging);
     for (DevBuf *b : {&c->x, &c->act, &c->act2, &c->out, &c->gate, &c->up, &c->h, &c->hr, &c->res, &c->pre, &c->sk, &c->lora})
         if (b->p) (void)hipFree(b->p);
     if (c->err) (void)hipFree(c->err);
@@ -609,8 +615,7 @@ static int project_q8k_host(prism_hip_ctx *c, prism_weight_id wid, const prism_q
     rc = ensure(c, c->act, ab);
     if (!rc) rc = ensure(c, c->out, sizeof(float) * n);
     if (!rc) {
-        hipError_t e = hipMemcpyAsync(c->act.p, act, ab, hipMemcpyHostToDevice, c->stream);
-        rc = e == hipSuccess ? PRISM_OK : hip_fail(c, e, "upload activations");
+        rc = upload(c, c->act.p, act, ab, c->stream, "upload activations");
     }
     if (!rc) rc = matvec(c, *w, kActQ8K, c->act.p, tokens, fused, static_cast<float *>(c->out.p), c->stream);
     if (!rc) rc = finish(c, out, static_cast<float *>(c->out.p), n);
@@ -642,8 +647,7 @@ static int project_q8_host(prism_hip_ctx *c, prism_weight_id wid, const prism_q8
     rc = ensure(c, c->act, ab);
     if (!rc) rc = ensure(c, c->out, sizeof(float) * n);
     if (!rc) {
-        hipError_t e = hipMemcpyAsync(c->act.p, act, ab, hipMemcpyHostToDevice, c->stream);
-        rc = e == hipSuccess ? PRISM_OK : hip_fail(c, e, "upload activations");
+        rc = upload(c, c->act.p, act, ab, c->stream, "upload activations");
     }
     if (!rc) rc = matvec(c, *w, kActQ8, c->act.p, tokens, pinned, static_cast<float *>(c->out.p), c->stream);
     if (!rc) rc = finish(c, out, static_cast<float *>(c->out.p), n);
@@ -675,8 +679,7 @@ static int project_f32_checked(prism_hip_ctx *c, prism_weight_id wid, const floa
     rc = ensure(c, c->x, sizeof(float) * w->cols * tokens);
     if (!rc) rc = ensure(c, c->out, sizeof(float) * n);
     if (!rc) {
-        hipError_t e = hipMemcpyAsync(c->x.p, x, sizeof(float) * w->cols * tokens, hipMemcpyHostToDevice, c->stream);
-        rc = e == hipSuccess ? PRISM_OK : hip_fail(c, e, "upload activations");
+        rc = upload(c, c->x.p, x, sizeof(float) * w->cols * tokens, c->stream, "upload activations");
     }
     if (!rc)
         rc = project_f32_dev(c, *w, static_cast<float *>(c->x.p), tokens, pinned, static_cast<float *>(c->out.p),
@@ -738,8 +741,7 @@ static int group_checked(prism_hip_ctx *c, const prism_weight_id *ws, uint32_t n
     rc = ensure(c, c->x, sizeof(float) * cols * tokens);
     if (!rc) rc = ensure(c, c->out, sizeof(float) * total * tokens);
     if (!rc) {
-        hipError_t e = hipMemcpyAsync(c->x.p, x, sizeof(float) * cols * tokens, hipMemcpyHostToDevice, c->stream);
-        rc = e == hipSuccess ? PRISM_OK : hip_fail(c, e, "upload activations");
+        rc = upload(c, c->x.p, x, sizeof(float) * cols * tokens, c->stream, "upload activations");
     }
     float *dev_out[8];
     uint64_t off = 0;
@@ -749,9 +751,7 @@ static int group_checked(prism_hip_ctx *c, const prism_weight_id *ws, uint32_t n
     }
     if (!rc) rc = group_tokens_impl(c, w, n, static_cast<const float *>(c->x.p), tokens, pinned, dev_out, c->stream);
     for (uint32_t i = 0; i < n && !rc; ++i) {
-        hipError_t e = hipMemcpyAsync(outs[i], dev_out[i], sizeof(float) * w[i]->rows * tokens, hipMemcpyDeviceToHost,
-                                      c->stream);
-        if (e != hipSuccess) rc = hip_fail(c, e, "copy group output");
+        rc = download(c, outs[i], dev_out[i], sizeof(float) * w[i]->rows * tokens, c->stream, "copy group output");
     }
     if (!rc) rc = drain(c, c->stream);
     return rc ? clear(rc) : rc;
@@ -817,18 +817,32 @@ static int ffn_checked(prism_hip_ctx *c, prism_weight_id gid, prism_weight_id ui
     rc = ensure(c, c->x, sizeof(float) * nx);
     if (!rc) rc = ensure(c, c->out, sizeof(float) * nout);
     if (!rc && residual) rc = ensure(c, c->res, sizeof(float) * nout);
-    if (!rc) {
-        hipError_t e = hipMemcpyAsync(c->x.p, x, sizeof(float) * nx, hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess && residual)
-            e = hipMemcpyAsync(c->res.p, residual, sizeof(float) * nout, hipMemcpyHostToDevice, c->stream);
-        rc = e == hipSuccess ? PRISM_OK : hip_fail(c, e, "upload activations");
-    }
+    if (!rc) rc = upload(c, c->x.p, x, sizeof(float) * nx, c->stream, "upload activations");
+    // The residual is first read by the down projection: a large one crosses on the side stream
+    // while gate and up run (every earlier user of its buffer was drained by its own call; 333
+    // tokens of 2048: 540 -> 453 us).  A small one goes first: behind queued kernels the runtime
+    // would wait for them (40 tokens: 164 / 173).
+    const size_t rbytes = sizeof(float) * nout;
+    const bool beside = residual && tokens > 1 && rbytes >= kSideMin && staging_ready(c);
+    auto residual_upload = [&]() -> int {
+        Staging &st = c->staging;
+        const int urc = upload(c, c->res.p, residual, rbytes, st.side, "upload residual", 0);
+        if (urc) return urc;
+        HIP_OR_FAIL(c, hipEventRecord(st.side_done, st.side));
+        HIP_OR_FAIL(c, hipStreamWaitEvent(c->stream, st.side_done, 0));
+        return PRISM_OK;
+    };
+    if (!rc && residual && !beside) rc = upload(c, c->res.p, residual, rbytes, c->stream, "upload residual");
     if (!rc)
         rc = ffn_tokens_impl(c, *g, *u, d, static_cast<float *>(c->x.p),
                              residual ? static_cast<float *>(c->res.p) : nullptr, tokens, pinned,
-                             static_cast<float *>(c->out.p), nullptr, c->stream, hb);
+                             static_cast<float *>(c->out.p), nullptr, c->stream, hb,
+                             beside ? std::function<int()>(residual_upload) : nullptr);
     if (!rc) rc = finish(c, out, static_cast<float *>(c->out.p), nout);
-    if (rc) zero(out, nout);
+    if (rc) {
+        if (c->staging.side) (void)hipStreamSynchronize(c->staging.side);  // no upload outlives a failed call
+        zero(out, nout);
+    }
     return rc;
 }
 

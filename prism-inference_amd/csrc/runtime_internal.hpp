@@ -53,6 +53,26 @@ inline int contract_for(uint32_t kind, uint64_t cols, int pinned) {
 
 }  // namespace prism::rt
 
+namespace prism::rt {
+
+// Pinned host memory the context's large host transfers pass through, kStageSlots pieces of
+// kStageBytes each (6 MiB in all), allocated by the first such transfer and freed with the
+// context, and a second stream for an upload that may run beside kernels.
+constexpr uint32_t kStageSlots = 4;
+constexpr size_t kStageBytes = 1536 * 1024;
+constexpr size_t kStageMin = 4u << 20;  // arrays on the context stream from here (see upload)
+constexpr size_t kSideMin = 1u << 20;   // an FFN residual on the side stream from here
+struct Staging {
+    uint8_t *mem = nullptr;
+    hipEvent_t done[kStageSlots] = {};  // the slot's last transfer
+    hipEvent_t side_done = nullptr;
+    hipStream_t side = nullptr;
+    uint32_t next = 0;
+    bool unavailable = false;  // an allocation failed: pageable transfers from then on
+};
+
+}  // namespace prism::rt
+
 struct prism_hip_ctx {
     int device = 0;
     uint32_t cus = 256;
@@ -73,6 +93,7 @@ struct prism_hip_ctx {
     prism_hip_statistics stats = {};
     prism_hip_diagnostics diag = {};
     const int32_t *cancel = nullptr;  // the request owner's cancellation flag, if any
+    prism::rt::Staging staging;
 };
 
 namespace prism {
@@ -252,6 +273,96 @@ struct Tally {
 inline const Weight *find(prism_hip_ctx *c, prism_weight_id w) {
     auto it = c->weights.find(w);
     return it == c->weights.end() ? nullptr : &it->second;
+}
+
+inline void staging_free(Staging &st) {
+    for (hipEvent_t &e : st.done)
+        if (e) (void)hipEventDestroy(e);
+    if (st.side_done) (void)hipEventDestroy(st.side_done);
+    if (st.side) (void)hipStreamDestroy(st.side);
+    if (st.mem) (void)hipHostFree(st.mem);
+    st = Staging{};
+}
+inline bool staging_ready(prism_hip_ctx *c) {
+    Staging &st = c->staging;
+    if (st.mem) return true;
+    if (st.unavailable) return false;
+    bool ok = hipHostMalloc(reinterpret_cast<void **>(&st.mem), kStageSlots * kStageBytes, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t &e : st.done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    ok = ok && hipEventCreateWithFlags(&st.side_done, hipEventDisableTiming) == hipSuccess;
+    ok = ok && hipStreamCreateWithFlags(&st.side, hipStreamNonBlocking) == hipSuccess;
+    if (ok) return true;
+    (void)hipGetLastError();
+    staging_free(st);
+    st.unavailable = true;
+    return false;
+}
+
+// Memory HIP knows nothing of (neither pinned nor device memory, which it transfers directly).
+inline bool pageable(const void *p) {
+    hipPointerAttribute_t a;
+    const bool known = hipPointerGetAttributes(&a, p) == hipSuccess && a.type != hipMemoryTypeUnregistered;
+    if (!known) (void)hipGetLastError();
+    return !known;
+}
+
+// A host array to the device on stream s.  The runtime stages pageable memory itself, one
+// piece after the other (2.7 MB: 100 us up, 146 us down, where the link takes 56 from pinned
+// memory and the copy to it 35), so large arrays pass through the context's pinned slots, the
+// copy of one piece beside the transfer of the one before.  Every piece costs some ten
+// microseconds of calls: the FFN chain without residual over 333 / 700 / 1000 tokens of 2048
+// (2.7 / 5.7 / 8.2 MB each way) took 469 / 838 / 1089 us, staged 464 / 748 / 988, and 200 tokens
+// 327 / 352; 512 KiB pieces gained nothing at 2.7 MB (394 / 422).  The array is read before the
+// call returns.
+inline int upload(prism_hip_ctx *c, void *dev, const void *host, size_t bytes, hipStream_t s, const char *what,
+                  size_t least = kStageMin) {
+    hipError_t e = hipSuccess;
+    if (bytes < least || !pageable(host) || !staging_ready(c)) {
+        e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+        return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
+    }
+    Staging &st = c->staging;
+    for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageBytes) {
+        const size_t n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
+        const uint32_t k = st.next++ % kStageSlots;
+        uint8_t *slot = st.mem + k * kStageBytes;
+        e = hipEventSynchronize(st.done[k]);  // returns at once for an event never recorded
+        if (e != hipSuccess) break;
+        std::memcpy(slot, static_cast<const uint8_t *>(host) + at, n);
+        e = hipMemcpyAsync(static_cast<uint8_t *>(dev) + at, slot, n, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess) e = hipEventRecord(st.done[k], s);
+    }
+    return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
+}
+// The other way; the host array is complete when the call returns (or, not staged, when the
+// stream drains).
+inline int download(prism_hip_ctx *c, void *host, const void *dev, size_t bytes, hipStream_t s, const char *what) {
+    hipError_t e = hipSuccess;
+    if (bytes < kStageMin || !pageable(host) || !staging_ready(c)) {
+        e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
+    }
+    Staging &st = c->staging;
+    const size_t pieces = (bytes + kStageBytes - 1) / kStageBytes;
+    const uint32_t first = st.next;
+    auto take = [&](size_t i) {  // piece i from its slot
+        const uint32_t k = (first + static_cast<uint32_t>(i)) % kStageSlots;
+        const size_t at = i * kStageBytes, n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
+        const hipError_t we = hipEventSynchronize(st.done[k]);
+        if (we == hipSuccess) std::memcpy(static_cast<uint8_t *>(host) + at, st.mem + k * kStageBytes, n);
+        return we;
+    };
+    for (size_t i = 0; i < pieces && e == hipSuccess; ++i) {
+        const uint32_t k = (first + static_cast<uint32_t>(i)) % kStageSlots;
+        const size_t at = i * kStageBytes, n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
+        e = i < kStageSlots ? hipEventSynchronize(st.done[k]) : take(i - kStageSlots);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(st.mem + k * kStageBytes, static_cast<const uint8_t *>(dev) + at, n, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(st.done[k], s);
+        ++st.next;
+    }
+    for (size_t i = pieces > kStageSlots ? pieces - kStageSlots : 0; i < pieces && e == hipSuccess; ++i) e = take(i);
+    return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
 }
 
 // Reads and clears the device error flag after the stream drained.
