@@ -3323,7 +3323,10 @@ SkinnyPlan skinny_plan(const MatvecArgs &a) {
     if (pl.sw) {
         const uint64_t room = a.scratch_fit / skinny_chunk_bytes<O>(a);
         if (pl.most > room) pl.most = room < 4 ? 4u : static_cast<uint32_t>(room);
-        if (a.rows < kSkinnyMinRows && (chunks < pl.most ? chunks : pl.most) > room) pl.sw = false;
+        // Calls that needed no such scratch before they came here (few rows; two or three pinned
+        // PTQ1 tokens) gather where it does not fit.
+        const bool was_scratch_free = a.rows < kSkinnyMinRows || (O == Op::PTQ1_PINNED && a.tokens <= 3);
+        if (was_scratch_free && (chunks < pl.most ? chunks : pl.most) > room) pl.sw = false;
     }
     return pl;
 }

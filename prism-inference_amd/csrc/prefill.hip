@@ -26,8 +26,8 @@
 // The activation side is prepared once per call by k_prefill_prep: Q8_0 quantization per
 // token, the codes stored as binary16 in operand order and the f32 scales beside them.
 //
-// The pinned contract (dot_q8_groups_pinned) runs k_prefill_ptq1_pinned on the same
-// tiles with its own operand order, four K=8 MFMAs per group (one per native lane) and
+// The pinned contract (dot_q8_groups_pinned) runs k_prefill_ptq1_pinned on tiles of 64 rows by
+// 64 tokens with its own operand order, four K=8 MFMAs per group (one per native lane) and
 // four FMA chains per output; see there.
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -799,8 +799,8 @@ size_t prefill_scratch_bytes(uint32_t kind, uint64_t cols, uint32_t tokens) {
     return ((Mp * cols * 2 + 255) & ~size_t(255)) + Mp * (cols / 32) * 4;
 }
 
-// Tokens from which PTQ1 takes the GEMM rather than the skinny kernel (up to four 16-token
-// chunks side by side per launch, each unit decoded once per chunk).  Measured (f32 input
+// Tokens from which PTQ1 can take the GEMM rather than the skinny kernel (16-token chunks side
+// by side, each unit decoded once per chunk); few rows stay there longer (skinny_beats_gemm).  Measured (f32 input
 // with its quantization, GEMM / skinny, us): 16 tokens 6144 x 2048 18.9 / 13.9, 12288 x 4096
 // 30.2 / 20.9, 151936 x 4096 139 / 93; 32 tokens source 6144 x 2048 20.0 / 17.3, 12288 x 4096
 // 31.6 / 31.8, 17408 x 5120 38.2 / 46.6, 32768 x 4096 41.7 / 54.8; pinned 6144 x 2048 31.6 /

@@ -641,8 +641,8 @@ size_t prefill_k_scratch_bytes(uint64_t cols, uint32_t tokens) {
     return align256(Mp * cols) + align256(nu * Mp * 4 * 8) + nu * Mp * 32;
 }
 
-// Tokens from which the GEMM takes over from the skinny kernel, which runs up to four
-// 16-token chunks side by side per launch.  Measured (f32 input with its quantization, us,
+// Tokens from which the GEMM can take over from the skinny kernel (16-token chunks side by
+// side); few rows stay there longer (skinny_beats_gemm).  Measured (f32 input with its quantization, us,
 // skinny / GEMM):
 // - below 8192 rows the skinny kernel stays ahead to 64 tokens (6144 x 2048, 48 tokens: Q2_K
 //   10.8 / 17.6, PQ2 14.1 / 15.6, Q8_0 16.8 / 23.7, TQ2_0 10.2 / 14.4; 64 tokens: Q2_K 12.1 /

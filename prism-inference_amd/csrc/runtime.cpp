@@ -61,6 +61,16 @@ int project_f32_dev(prism_hip_ctx *c, const Weight &w, const float *x, uint32_t 
         if (prepared) {
             const size_t need = act_bytes(contract_for(w.kind, w.cols, pinned), w.cols, tokens);
             a.act_fit = need <= scratch_room(c, sc, role, need);
+            if (a.act_fit && tokens > 1 && w.rows < 1024) {
+                // Below 1024 rows the prologue path needs no scratch: what a batch kernel on
+                // prepared blocks needs beside them must fit too (a fixed region bounds the
+                // kernel choice itself, run_matvec).
+                MatvecArgs pa = matvec_args(c, w, a.qcontract_is_q8k ? kActQ8K : kActQ8, nullptr, tokens, pinned, out, s);
+                size_t more = tiled_scratch_bytes(pa);
+                pa.scratch_fit = scratch_room(c, sc, c->sk, more);
+                if (more > pa.scratch_fit) more = tiled_scratch_bytes(pa);
+                a.act_fit = (sc && sc->base) || more <= pa.scratch_fit;
+            }
             if (!a.act_fit) prepared = tiled_needs_prepared(a);
         }
         if (!prepared) return run_matvec(c, a, true, &scr);

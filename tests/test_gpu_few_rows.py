@@ -99,3 +99,32 @@ def test_gpu_few_rows_keep_the_scratch_free_path():
                 g.launch()
                 assert d.sync() == 0
                 assert np.array_equal(out.to_numpy(np.uint32), b.to_numpy(np.uint32)[:rows * 3])
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens,pinned", [
+    (ph.KIND_PTQ1, 200, 8192, 3, False),   # split-K with scratch
+    (ph.KIND_PTQ1, 8200, 6144, 2, True),   # lane-ordered copy, prepared blocks only
+    (ph.KIND_Q8_0, 500, 2048, 12, True),   # lane-ordered copy
+    (ph.KIND_PTQ1, 8200, 5120, 1, False),  # a quantizer of its own: one token
+    (ph.KIND_PTQ1, 8256, 4096, 1, True)])  # the stream form: one token
+def test_gpu_first_call_under_capture(kind, rows, cols, tokens, pinned):
+    """The first call of a context may be captured where its former path needed no scratch: it
+    gives the same bits as an uncaptured call."""
+    import hiprt
+
+    w = synth.weights(kind, rows, cols, seed=9)
+    X = np.ascontiguousarray(synth.activations(cols, seed=10, tokens=tokens).reshape(tokens, cols), np.float32)
+    with ph.Context(0) as c, ph.Context(0) as d:
+        wc, wd = c.weight(kind, cols, rows, w), d.weight(kind, cols, rows, w)
+        x, a, b = DeviceBuffer.from_numpy(X), DeviceBuffer(rows * tokens * 4), DeviceBuffer(rows * tokens * 4)
+        path, inp = ph.PATH_F32, x
+        if kind == ph.KIND_PTQ1 and pinned and tokens > 1:
+            path, inp = ph.PATH_Q8, DeviceBuffer(tokens * cols // 32 * 40)
+            c.quantize_q8_device(x, cols, tokens, ph.Q8_PINNED_NATIVE, inp)
+        c.project_device(wc, path, inp, tokens, pinned, a)
+        assert c.sync() == 0
+        g = hiprt.Graph(d.stream(), lambda: d.project_device(wd, path, inp, tokens, pinned, b))
+        for _ in range(3):
+            g.launch()
+            assert d.sync() == 0
+            assert np.array_equal(a.to_numpy(np.uint32), b.to_numpy(np.uint32))
