@@ -828,12 +828,15 @@ static int ffn_checked(prism_hip_ctx *c, prism_weight_id gid, prism_weight_id ui
     if (!rc) rc = ensure(c, c->out, sizeof(float) * nout);
     if (!rc && residual) rc = ensure(c, c->res, sizeof(float) * nout);
     if (!rc) rc = upload(c, c->x.p, x, sizeof(float) * nx, c->stream, "upload activations");
-    // The residual is first read by the down projection: a large one crosses on the side stream
-    // while gate and up run (every earlier user of its buffer was drained by its own call; 333
-    // tokens of 2048: 540 -> 453 us).  A small one goes first: behind queued kernels the runtime
-    // would wait for them (40 tokens: 164 / 173).
+    // The residual is first read by the down projection: a large pageable one crosses on the side
+    // stream while gate and up run (every earlier user of its buffer was drained by its own call;
+    // 333 tokens of 2048: 540 -> 453 us).  A small one goes first: behind queued kernels the
+    // runtime would wait for them (40 tokens: 164 / 173).  So does pinned or device memory, which
+    // HIP reads when the copy's turn comes and not before the call returns: the caller may have
+    // filled it by work queued on the context stream (or on the null stream, which orders itself
+    // with the context stream but not with the side stream), so its copy stays on that stream.
     const size_t rbytes = sizeof(float) * nout;
-    const bool beside = residual && tokens > 1 && rbytes >= kSideMin && staging_ready(c);
+    const bool beside = residual && tokens > 1 && rbytes >= kSideMin && pageable(residual) && staging_ready(c);
     auto residual_upload = [&]() -> int {
         Staging &st = c->staging;
         const int urc = upload(c, c->res.p, residual, rbytes, st.side, "upload residual", 0);

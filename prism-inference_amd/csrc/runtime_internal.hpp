@@ -61,7 +61,7 @@ namespace prism::rt {
 constexpr uint32_t kStageSlots = 4;
 constexpr size_t kStageBytes = 1536 * 1024;
 constexpr size_t kStageMin = 4u << 20;  // arrays on the context stream from here (see upload)
-constexpr size_t kSideMin = 1u << 20;   // an FFN residual on the side stream from here
+constexpr size_t kSideMin = 1u << 20;   // a pageable FFN residual on the side stream from here
 struct Staging {
     uint8_t *mem = nullptr;
     hipEvent_t done[kStageSlots] = {};  // the slot's last transfer

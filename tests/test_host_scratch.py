@@ -1,0 +1,82 @@
+"""The library's host side on the CPU: libprism_hip.so over a HIP runtime without a device
+(hip_stub.cpp), which writes down allocations, copies and launches and runs no kernel.  Covers
+what no result shows: the stream an array is copied on, and what a graph may hold.
+"""
+
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+LIB = os.path.join(ROOT, "prism-inference_amd", "libprism_hip.so")
+
+PRELUDE = """
+import ctypes, sys
+import numpy as np
+S = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+S.stub_log.restype = ctypes.c_char_p
+S.stub_largest.argtypes = [ctypes.c_size_t]
+S.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
+S.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+sys.path.insert(0, sys.argv[2])
+import prism_hip as ph
+P, L = ctypes.c_void_p, ph.lib()
+X, OUT = P(0x10000000), P(0x20000000)  # device arrays of the caller; nothing reads them
+def log():
+    return S.stub_log().decode().splitlines()
+def weight(c, kind, cols, rows):
+    return L.prism_hip_weight_wrap_tiled(c, kind, cols, rows, P(0x70000000), L.prism_hip_weight_tiled_bytes(c, kind, cols, rows))
+def project(c, w, path, tokens, pinned):
+    return L.prism_hip_project_device(c, w, path, X, tokens, int(pinned), OUT, None)
+def captured(call):
+    S.stub_capture(1)
+    rc = call()
+    S.stub_capture(0)
+    return rc
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", so], check=True)
+
+    def run(code, *args):
+        src = PRELUDE + textwrap.dedent(code)
+        p = subprocess.run([sys.executable, "-c", src, so, os.path.dirname(LIB), *map(str, args)], capture_output=True,
+                           text=True, timeout=300)
+        assert p.returncode == 0, p.stdout + p.stderr
+        return p.stdout
+
+    return run
+
+
+@pytest.mark.parametrize("memory", ["pinned", "device", "pageable"])
+def test_ffn_residual_is_copied_behind_the_callers_work(stub, memory):
+    """Memory HIP reads when the copy's turn comes is copied on the context stream, where the caller
+    orders its work; only pageable memory, read before the call returns, may take another."""
+    stub("""
+        c = L.prism_hip_create(0, 0, 0)
+        hidden, ffn, tokens = 1024, 1536, 300
+        g, u, d = weight(c, ph.KIND_PTQ1, hidden, ffn), weight(c, ph.KIND_PTQ1, hidden, ffn), weight(c, ph.KIND_PTQ1, ffn, hidden)
+        n = tokens * hidden * 4
+        keep = [np.zeros(tokens * hidden, np.float32) for _ in range(3)]
+        x, res, out = (P(a.ctypes.data) for a in keep)
+        if sys.argv[3] != "pageable":
+            res = P()
+            assert (S.hipHostMalloc(ctypes.byref(res), n, 0) if sys.argv[3] == "pinned" else S.hipMalloc(ctypes.byref(res), n)) == 0
+        log()
+        assert L.prism_hip_ffn_chain_tokens(c, g, u, d, x, res, tokens, 0, 0, out) == 0
+        stream = "stream " + hex(L.prism_hip_stream(c))
+        copies = [l for l in log() if l.startswith("copy ")]
+        if sys.argv[3] == "pageable":
+            assert any(not l.endswith(stream) for l in copies), copies
+        else:
+            assert all(l.endswith(stream) for l in copies) and any(f"<- {hex(res.value)} " in l for l in copies), copies
+        L.prism_hip_destroy(c)
+        """, memory)
