@@ -28,12 +28,15 @@ bool gemm_path(prism_hip_ctx *c, const Weight &w, uint32_t tokens, int pinned, c
     if (!w.tiled || tokens < kPrefillMinTokens || !prefill_supported(w.kind, w.cols, w.rows, pinned, tokens)) return false;
     const int contract = contract_for(w.kind, w.cols, pinned);
     MatvecArgs a = matvec_args(c, w, contract == 0 ? kActQ8K : kActQ8, nullptr, tokens, pinned, nullptr, c->stream);
-    const size_t act = (act_bytes(contract, w.cols, tokens) + 255) & ~size_t(255);
+    const size_t act = act_bytes(contract, w.cols, tokens);  // as project_f32_dev asks for them
     a.residual = residual;
     if (!skinny_beats_gemm(a)) return true;
     if (act > scratch_room(c, sc, role, act)) return true;
     a.scratch_fit = scratch_room(c, sc, c->sk, tiled_scratch_bytes(a));
-    if (sc && sc->base) a.scratch_fit -= act;  // one region holds both
+    if (sc && sc->base) {  // one region holds both, each 256-byte aligned
+        const size_t taken = (act + 255) & ~size_t(255);
+        a.scratch_fit = a.scratch_fit > taken ? a.scratch_fit - taken : 0;
+    }
     return !skinny_beats_gemm(a);
 }
 

@@ -80,3 +80,33 @@ def test_ffn_residual_is_copied_behind_the_callers_work(stub, memory):
             assert all(l.endswith(stream) for l in copies) and any(f"<- {hex(res.value)} " in l for l in copies), copies
         L.prism_hip_destroy(c)
         """, memory)
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_a_call_made_once_uncaptured_can_be_captured(stub, seed):
+    """Every form of a device call, at sizes on all routes: scratch never grows under capture, and one
+    uncaptured call of the same arguments is all that a capture needs.  Both take the same kernels."""
+    stub("""
+        import random
+        rng = random.Random(int(sys.argv[3]))
+        kinds = [ph.KIND_PTQ1, ph.KIND_PQ2, ph.KIND_Q2_K, ph.KIND_Q8_0, ph.KIND_TQ1_0, ph.KIND_TQ2_0]
+        launches = lambda: [l.split(" stream")[0] for l in log() if l.startswith("launch ")]
+        for i in range(3000):
+            kind = kinds[i % 6]
+            unit = ph.LAYOUT[kind][0] if kind not in (ph.KIND_Q8_0,) else 128
+            rows = int(2 ** rng.uniform(0, 10 if i % 2 else 17))
+            cols = max(1, int(2 ** rng.uniform(7, 14.2)) // unit) * unit
+            tokens = rng.choice([1, 2, 3, rng.randint(4, 16), rng.randint(17, 600), rng.randint(17, 600)])
+            pinned = rng.random() < 0.5
+            q8k = kind in (ph.KIND_Q2_K, ph.KIND_TQ1_0, ph.KIND_TQ2_0) or (kind == ph.KIND_PQ2 and cols % 256 == 0)
+            path = rng.choice([ph.PATH_F32, ph.PATH_Q8K if q8k else ph.PATH_Q8])
+            c = L.prism_hip_create(0, 0, 0)
+            w = weight(c, kind, cols, rows)
+            log()
+            case = (kind, rows, cols, tokens, pinned, path)
+            assert project(c, w, path, tokens, pinned) == 0, case
+            eager = launches()
+            assert captured(lambda: project(c, w, path, tokens, pinned)) == 0, (case, L.prism_hip_last_error(c))
+            assert launches() == eager, case
+            L.prism_hip_destroy(c)
+        """, seed)
