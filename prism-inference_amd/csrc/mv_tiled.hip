@@ -3282,6 +3282,8 @@ struct SkinnyPlan {
 // 16-row blocks of a matrix, one skinny workgroup each.
 uint64_t skinny_blocks(uint64_t rows) { return (rows + kTile - 1) / kTile * 4; }
 
+constexpr uint64_t kSkinnyCopyBytes = 32ull << 20;
+
 template <Op O>
 size_t skinny_chunk_bytes(const MatvecArgs &a) {
     return a.cols / unit_weights<O>() * 64u * (sk_lane_bytes<O>() + 4u);
@@ -3318,9 +3320,13 @@ SkinnyPlan skinny_plan(const MatvecArgs &a) {
     // The chunks of a launch run side by side (grid y), each a batch of its own, so several fill
     // the chip where one leaves it latency-bound (PQ2 1003 x 8320, 338 tokens, us: 4 / 8 / 16 /
     // 24 chunks a launch 82 / 53 / 45 / 34).  Thirty-two keep the lane-ordered copies of rows of
-    // up to 17408 inputs under 12 MB; a scratch that holds fewer takes fewer.
+    // up to 17408 inputs under 12 MB; past kSkinnyCopyBytes (58000 inputs) they stop growing with
+    // the row, down to the four chunks every scratch was asked for, and a scratch that holds fewer
+    // takes fewer.
     pl.most = 32;
     if (pl.sw) {
+        const uint64_t bounded = kSkinnyCopyBytes / skinny_chunk_bytes<O>(a);
+        if (pl.most > bounded) pl.most = bounded < 4 ? 4u : static_cast<uint32_t>(bounded);
         const uint64_t room = a.scratch_fit / skinny_chunk_bytes<O>(a);
         if (pl.most > room) pl.most = room < 4 ? 4u : static_cast<uint32_t>(room);
         // Calls that needed no such scratch before they came here (few rows; two or three pinned
@@ -3740,7 +3746,12 @@ size_t tiled_scratch_bytes(const MatvecArgs &a) {
     if (a.act_format != kActF32 && !token_by_token(a) && gemm_eligible(a))
         return prefill_scratch_bytes(a.kind, a.cols, a.tokens);
     if (!skinny_eligible(a)) return 0;
-    return static_cast<size_t>(dispatch(a, [&]<Op O>() { return static_cast<int>(skinny_scratch<O>(a)); }));
+    size_t bytes = 0;  // not dispatch's int: the copies of 3.7 million inputs pass 2 GiB
+    dispatch(a, [&]<Op O>() {
+        bytes = skinny_scratch<O>(a);
+        return 0;
+    });
+    return bytes;
 }
 
 bool tiled_prologue_fits(const MatvecArgs &a) {

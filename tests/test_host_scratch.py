@@ -110,3 +110,24 @@ def test_a_call_made_once_uncaptured_can_be_captured(stub, seed):
             assert launches() == eager, case
             L.prism_hip_destroy(c)
         """, seed)
+
+
+@pytest.mark.parametrize("cols,tokens", [(65536, 520), (1 << 20, 512), (3959808, 65), (3959808, 2750), (30000128, 600)])
+def test_scratch_of_very_long_rows(stub, cols, tokens):
+    """The lane-ordered copies stay bounded, and their size is not cut to 32 bits: 32 chunks of 3.7
+    million inputs, or four of 30 million, pass 2 GiB."""
+    stub("""
+        cols, tokens = int(sys.argv[3]), int(sys.argv[4])
+        for kind, unit in ((ph.KIND_Q8_0, 128), (ph.KIND_PQ2, 128), (ph.KIND_PTQ1, 128), (ph.KIND_TQ1_0, 256)):
+            for rows in (97, 2100):
+                c = L.prism_hip_create(0, 0, 0)
+                w = weight(c, kind, cols // unit * unit, rows)
+                log()
+                assert project(c, w, ph.PATH_F32, tokens, False) == 0, (kind, rows, L.prism_hip_last_error(c))
+                sizes = [int(l.split()[2]) for l in log() if l.startswith("malloc ")]
+                copies = max(32 << 20, 4 * (cols // 128 + 1) * 64 * 68)  # four chunks, at most 64 + 4 bytes a lane
+                blocks = tokens * cols // 32 * 40  # the prepared activations: Q8_0, larger than Q8_K
+                gemm = (tokens + 127) // 128 * 128 * cols * 3
+                assert len(sizes) <= 2 and sum(sizes) <= max(blocks + copies, gemm) + 8192, (kind, rows, sizes)
+                L.prism_hip_destroy(c)
+        """, cols, tokens)
