@@ -372,6 +372,7 @@ void prism_hip_destroy(prism_hip_ctx *c) {
     staging_free(c->staging);
     for (DevBuf *b : {&c->x, &c->act, &c->act2, &c->out, &c->gate, &c->up, &c->h, &c->hr, &c->res, &c->pre, &c->sk, &c->lora})
         if (b->p) (void)hipFree(b->p);
+    for (void *p : c->retired) (void)hipFree(p);
     if (c->err) (void)hipFree(c->err);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1021,6 +1022,7 @@ static int project_device_checked(prism_hip_ctx *c, prism_weight_id wid, int pat
 int prism_hip_project_device(prism_hip_ctx *c, prism_weight_id wid, int path, const void *act, uint32_t tokens,
                              int pinned, float *out, void *stream) {
     Tally t(c, 1, path == PRISM_PATH_F32);
+    CaptureNote note(c);
     return t(project_device_checked(c, wid, path, act, tokens, pinned, out, stream, t));
 }
 
@@ -1075,6 +1077,7 @@ int prism_hip_ffn_chain_device(prism_hip_ctx *c, prism_weight_id gid, prism_weig
                                const float *x, const float *residual, uint32_t hadamard_block, int pinned,
                                float *out, float *h, void *stream) {
     Tally t(c, did ? 3 : 2, true);
+    CaptureNote note(c);
     return t(ffn_device_checked(c, gid, uid, did, x, residual, hadamard_block, pinned, out, h, stream, t));
 }
 

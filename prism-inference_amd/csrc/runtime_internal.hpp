@@ -85,6 +85,10 @@ struct prism_hip_ctx {
     int64_t next_id = 1;
     int *err = nullptr;  // device error flag
     prism::rt::DevBuf x, act, act2, out, gate, up, h, hr, res, pre, sk, lora;
+    // Whether the current device call took one of them, whether a captured one ever did (a graph
+    // may hold any of them from then on), and those outgrown since, kept for such graphs.
+    bool scratch_used = false, scratch_captured = false;
+    std::vector<void *> retired;
     // This device's copy of the fixed scratch array (static_scratch.hip), looked up at
     // creation; nullptr if the lookup failed.
     void *noalloc = nullptr;
@@ -155,24 +159,62 @@ inline int launch_result(prism_hip_ctx *c, int rc, const char *what) {
         if (e_ != hipSuccess) return hip_fail(ctx, e_, #call); \
     } while (0)
 
+inline bool capturing(prism_hip_ctx *c) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
 // Grows a scratch buffer.  Work runs on the context stream only, so a capture in
 // progress there means the buffer is about to be baked into a graph: growing it would
 // free memory the graph already references, so that is refused (size the scratch with
-// one uncaptured call first).
+// one uncaptured call first).  Once a captured call has used scratch, an outgrown buffer is
+// kept until the context goes, since a graph may still write it at any replay; doubling then
+// keeps those of a role together below its current size.
 inline int ensure(prism_hip_ctx *c, DevBuf &b, size_t bytes) {
+    c->scratch_used = true;
     if (bytes <= b.cap) return PRISM_OK;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+    if (capturing(c))
         return fail(c, PRISM_ERR_UNSUPPORTED, "scratch would grow during graph capture: run the call once uncaptured");
+    size_t n = bytes < 4096 ? 4096 : bytes;
+    if (b.p && c->scratch_captured) {
+        void *p = nullptr;
+        const size_t twice = b.cap > n / 2 ? 2 * b.cap : n;
+        hipError_t e = hipMalloc(&p, twice);
+        if (e == hipSuccess) {
+            n = twice;
+        } else if (twice > n) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, n);
+        }
+        if (e != hipSuccess) return hip_fail(c, e, "hipMalloc(scratch)");
+        c->retired.push_back(b.p);
+        b.p = p;
+        b.cap = n;
+        return PRISM_OK;
+    }
     if (b.p) (void)hipFree(b.p);
     b.p = nullptr;
     b.cap = 0;
-    size_t n = bytes < 4096 ? 4096 : bytes;
     hipError_t e = hipMalloc(&b.p, n);
     if (e != hipSuccess) return hip_fail(c, e, "hipMalloc(scratch)");
     b.cap = n;
     return PRISM_OK;
 }
+
+// Around a device call, which a caller may capture: notes whether it put context scratch into a
+// graph.  Asked after the launches, where the capture query (about 0.4 us) costs an uncaptured
+// call nothing: the device is busy with them.
+struct CaptureNote {
+    prism_hip_ctx *c;
+    explicit CaptureNote(prism_hip_ctx *ctx) : c(ctx) {
+        if (c) c->scratch_used = false;
+    }
+    ~CaptureNote() {
+        if (c && c->scratch_used && !c->scratch_captured) c->scratch_captured = capturing(c);
+    }
+    CaptureNote(const CaptureNote &) = delete;
+    CaptureNote &operator=(const CaptureNote &) = delete;
+};
 
 // The stream a device-pointer call runs on.  The context's scratch buffers and error
 // flag are shared by all of its calls, so they are ordered on the one context stream;
@@ -423,9 +465,7 @@ inline size_t scratch_room(prism_hip_ctx *c, const Scratch *sc, const DevBuf &ro
         return at < sc->cap ? sc->cap - at : 0;
     }
     if (need <= role.cap) return ~size_t(0);
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
-    return capturing ? role.cap : ~size_t(0);
+    return capturing(c) ? role.cap : ~size_t(0);
 }
 
 // sc == nullptr: the context's grow-only buffers.

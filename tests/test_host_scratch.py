@@ -131,3 +131,61 @@ def test_scratch_of_very_long_rows(stub, cols, tokens):
                 assert len(sizes) <= 2 and sum(sizes) <= max(blocks + copies, gemm) + 8192, (kind, rows, sizes)
                 L.prism_hip_destroy(c)
         """, cols, tokens)
+
+
+CAPTURED = [  # kind, rows, cols, tokens, pinned, path, and the tokens of the call that outgrows its scratch
+    ("PTQ1", 5120, 17408, 1, False, "F32", 40), ("PQ2", 5120, 17408, 1, True, "F32", 40),  # a quantizer of its own
+    ("PTQ1", 8256, 4096, 1, True, "F32", 40),  # the stream form
+    ("Q2_K", 500, 2048, 7, False, "F32", 90), ("Q8_0", 500, 2048, 12, True, "F32", 90),  # few rows
+    ("PTQ1", 8200, 6144, 2, True, "Q8", 30), ("PTQ1", 6144, 2048, 64, False, "F32", 600),  # copies; a GEMM
+    ("PTQ1", 5120, 6144, 2, False, "Q8", 40)]  # split-K
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens,pinned,path,more", CAPTURED)
+@pytest.mark.parametrize("ffn", [False, True])
+def test_scratch_of_a_captured_call_outlives_larger_calls(stub, kind, rows, cols, tokens, pinned, path, more, ffn):
+    """Every buffer there was when a call was captured is still there after calls that need more, the
+    kept ones stay below the current ones, and the context gives all of them back."""
+    stub("""
+        kind, path = getattr(ph, "KIND_" + sys.argv[3]), getattr(ph, "PATH_" + sys.argv[8])
+        rows, cols, tokens, more, pinned, ffn = (int(a) for a in sys.argv[4:7] + sys.argv[9:10] + [sys.argv[7] == "True", sys.argv[10] == "True"])
+        c = L.prism_hip_create(0, 0, 0)
+        empty = S.stub_allocations()
+        w = weight(c, kind, cols, rows)
+        g, u, d = weight(c, kind, cols, 8192), weight(c, kind, cols, 8192), weight(c, kind, 8192, cols)
+        def call():
+            if ffn:
+                return L.prism_hip_ffn_chain_device(c, g, u, d, X, None, 64, int(pinned), OUT, None, None)
+            return project(c, w, path, tokens, pinned)
+        assert call() == 0
+        log()
+        # Uncaptured so far: an outgrown buffer is given back at once.
+        assert project(c, w, path, tokens + 1, pinned) == 0 and call() == 0
+        log()
+        assert captured(call) == 0
+        assert not any(l.startswith(("malloc", "free")) for l in log())
+        sizes = {}
+        def grow(t):
+            for k in (ph.PATH_F32, path):
+                assert project(c, w, k, t, pinned) == 0
+            for l in log():
+                f = l.split()
+                assert f[0] != "free", l
+                if f[0] == "malloc":
+                    sizes[f[1]] = int(f[2])
+        for t in range(more, more + 200):
+            grow(t)
+        assert sizes and len(sizes) <= 4 * 3, sizes  # doubling: few buffers a role
+        assert captured(lambda: project(c, w, path, more, pinned)) == 0
+        # Memory for the exact size only, and then none: the old buffer keeps serving.
+        big = 40 * more
+        need = max(sizes.values()) * 4
+        S.stub_largest(need)
+        while project(c, w, path, big, pinned) == 0 and big < 4000000:
+            big *= 2
+        assert big < 4000000
+        assert not any(l.startswith("free") for l in log())
+        assert call() == 0 and captured(call) == 0
+        L.prism_hip_destroy(c)
+        assert S.stub_allocations() == empty - 1, (S.stub_allocations(), empty)  # and the error flag
+        """, kind, rows, cols, tokens, pinned, path, more, ffn)
