@@ -243,6 +243,12 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
 }
 
+// No memory access of this wavefront moves across it, in either direction, in the compiler: the
+// waits that count loads rest on their order.  A plain load of memory that a __restrict__ argument
+// names is exempt (nothing else may write it, so the compiler moves it across barriers, waits and
+// this fence alike): kernels that count theirs take the pointer without.
+__device__ __forceinline__ void keep_order() { asm volatile("" ::: "memory"); }
+
 // 16 bytes to LDS, past the compiler's own bookkeeping: before an ordinary LDS store it waits
 // for every direct-to-LDS load in flight, whatever they write.  The next lds_barrier waits for it.
 __device__ __forceinline__ void lds_store16(u32x4 *p, u32x4 v) {
@@ -606,7 +612,7 @@ struct LaneDecoder {
 // are decoded into it, and one barrier a half hands both over (34 KiB, four workgroups a CU).
 template <bool HALF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_prefill_ptq1_pinned(
-    const uint8_t *__restrict__ W, uint32_t rows, uint32_t nu, const _Float16 *__restrict__ xh,
+    const uint8_t *W, uint32_t rows, uint32_t nu, const _Float16 *__restrict__ xh,
     const float *__restrict__ sc, uint32_t M, uint32_t Mp, uint32_t xcd_major, float *__restrict__ out,
     int *__restrict__ err) {
     constexpr uint32_t NT = kPinnedTokens;
@@ -649,10 +655,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 ((u * 32 + 16 * half + k + lane / 32) * Mp + t0 + 2 * (lane % 32)) * 8u, 0, 0, 0);
         }
     };
+    // Every wavefront a quarter, a dword per lane: all issue the same loads, outside any branch.
+    static_assert(NT * 16 == 4 * 64 * 4, "one dword of the scales per thread");
     auto stage_scales = [&](uint32_t u, float4 (&scl)[NT]) {
-        if (lane < NT / 4)  // every wavefront a quarter: all issue the same loads
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(&scl[wave * (NT / 4)]), 16,
-                                                     (u * Mp + t0 + wave * (NT / 4) + lane) * 16u, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(&scl[wave * (NT / 4)]), 4,
+                                                 (u * Mp + t0 + wave * (NT / 4)) * 16u + 4u * lane, 0, 0, 0);
     };
     // The dwords of LaneDecoder's half tw of the lane's row: A_tw, A_{tw+2}, B_tw and the tail.
     uint32_t raw[4];
@@ -712,9 +719,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     };
 
     // Half n = 2u + half is staged three halves ahead, into buffer n % 4.  Each wavefront issues,
-    // in this order, 2 loads in a first half (codes of half n + 3) and 7 in a second (2 of codes,
-    // 1 of scales, 4 of weights), also past the row's end (the buffers' bounds then yield zeros),
-    // so the loads still allowed in flight when half n + 1 must have landed are those counts.
+    // in this order (keep_order), 2 loads in a first half (codes of half n + 3) and 7 in a second (2
+    // of codes, 1 of scales, 4 of weights), also past the row's end (the buffers' bounds then yield
+    // zeros), so the loads still allowed in flight when half n + 1 must have landed are those counts.
     load(0);
     stage(0, 0, act0);
     stage_scales(0, scl0);
@@ -725,6 +732,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     stage_scales(1, scl1);
     load(1);
     decode(0, opa0);
+    keep_order();
     wait_vmcnt0();
     lds_barrier();
     auto block = [&](uint32_t u, const uint8_t (&a0)[16][kRun], const uint8_t (&a1)[16][kRun],
@@ -738,12 +746,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             const float s01[2] = {sg.x, sg.y};
             multiply(dw, s01, a0, opa0);
         }
+        keep_order();
         __builtin_amdgcn_s_waitcnt(0x0F79);  // vmcnt(9): half 2u + 1 has landed
         lds_barrier();
+        keep_order();
         // Second half, while the next block's first operands are made.
         const uint32_t d1 = dw;
         stage(u + 2, 0, n0);
         stage_scales(u + 2, scl);
+        keep_order();
         dw = h ? 0u : raw[3] >> 16;
         dec.start(raw, h);
         load(u + 2);
@@ -752,8 +763,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             const float s23[2] = {sg.z, sg.w};
             multiply(d1, s23, a1, opa1);
         }
+        keep_order();
         __builtin_amdgcn_s_waitcnt(0x0F7D);  // vmcnt(13): half 2u + 2 and its scales have landed
         lds_barrier();
+        keep_order();
     };
     for (uint32_t u = 0; u < nu; u += 2) {
         block(u, act0, act1, act0, act3, scl0);
