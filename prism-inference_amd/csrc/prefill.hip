@@ -46,6 +46,9 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr uint32_t kRowsPerWg = 128, kTokAlign = 128;
 constexpr uint32_t kPinnedTokens = 64;  // tokens per workgroup of the pinned GEMM
+// Where its workgroups are 128 rows by 32 tokens instead of 64 by 64: nowhere, in a last group of
+// at most 32 tokens, everywhere.
+constexpr uint32_t kPinnedAll64 = 0, kPinnedLast32 = 1, kPinnedAll32 = 2;
 
 constexpr uint32_t sel_bytes(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
     return b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
@@ -595,6 +598,121 @@ struct LaneDecoder {
     }
 };
 
+// dd[r] = fl(d_w * A_g.scale) for every (row, token) of a 32 x 32 tile, as an outer product: HALF
+// where this library's quantizer made the scales, which are binary16 values then; a caller's own
+// blocks may hold any binary32 scale (K = 2 with the second term zero, one rounding).  dw: the
+// lane's row scale (binary16 bits) in lanes 0..31, else 0.
+template <bool HALF>
+__device__ __forceinline__ v16f pinned_scale_products(uint32_t dw, float sg, uint32_t h) {
+    if constexpr (HALF)
+        return scale_products(dw, h ? 0u : __builtin_bit_cast(uint16_t, static_cast<_Float16>(sg)));
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x2f32(h2f(dw), h ? 0.0f : sg, v16f{}, 0, 0, 0);
+}
+
+// Token t's outputs of a wavefront's 32 rows, (L0 + L1) + (L2 + L3); yr: its row of the tile.
+__device__ __forceinline__ void pinned_store(const float (&L)[4][16], bool active, uint32_t t, uint32_t M, float *yr,
+                                             uint32_t out0, uint32_t trows, int *err) {
+    if (!active || t >= M) return;
+    bool bad = false;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t r = out0 + 8 * q + e;
+            if (r < trows) {
+                const int k = 4 * q + e;
+                const float v = (L[0][k] + L[1][k]) + (L[2][k] + L[3][k]);
+                yr[r] = v;
+                bad |= !finite(v);
+            }
+        }
+    }
+    if (bad) raise_error(err, kErrNonfinite);
+}
+
+// A workgroup of the last 32 tokens: 128 rows, every wavefront 32 of them with its own decode.
+template <bool HALF>
+__device__ __forceinline__ void pinned_tail(const uint8_t *W, uint32_t rows, uint32_t nu, __amdgpu_buffer_rsrc_t rx,
+                                            __amdgpu_buffer_rsrc_t rs, uint32_t M, uint32_t Mp, uint32_t t0, uint32_t bx,
+                                            float *out, int *err, uint8_t (&act0)[32][32 * 8], uint8_t (&act1)[32][32 * 8],
+                                            float4 (&scl0)[32], float4 (&scl1)[32]) {
+    constexpr uint32_t NT = 32, kRun = NT * 8;
+    const uint32_t lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = 2 * bx + (wave >> 1), hw = wave & 1;
+    const uint32_t tiles = (rows + kTile - 1) / kTile, row_bytes = nu * 28;
+    uint32_t trows = 0;
+    if (tile < tiles) {
+        const uint32_t left = rows - tile * kTile;
+        trows = left < kTile ? left : kTile;
+    }
+    const bool active = 32 * hw < trows;  // uniform per wavefront
+    const uint32_t trp = (trows + 7u) & ~7u;
+    const __amdgpu_buffer_rsrc_t rw =
+        make_rsrc(W + static_cast<size_t>(active ? tile : 0) * kTile * row_bytes, active ? trp * row_bytes : 0u);
+    const uint32_t row = 32 * hw + r32, out0 = 32 * hw + 4 * h;  // tile rows
+
+    // Block u's codes (32 runs of NT * 8 bytes; one instruction moves four, lane l tokens
+    // 2 (l % 16), + 1 of run l / 16) and the scales of the workgroup's tokens.
+    auto stage = [&](uint32_t u, uint8_t (&act)[32][kRun], float4 (&scl)[NT]) {
+        for (uint32_t i = wave; i < 8; i += 4)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void *)(&act[4 * i][0]), 16,
+                                                     ((u * 32 + 4 * i + lane / 16) * Mp + t0 + 2 * (lane % 16)) * 8u, 0,
+                                                     0, 0);
+        if (wave == 0 && lane < NT)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(&scl[0]), 16, (u * Mp + t0 + lane) * 16u, 0,
+                                                     0, 0);
+    };
+    float L[4][16];
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) L[l][r] = 0.0f;
+    const v16f zero = {};
+
+    RawBlock w = {};  // stays zero in an inactive wavefront
+    stage(0, act0, scl0);
+    if (active) load_block_codes(rw, 0, trp, row, w);
+    wait_vmcnt0();
+    lds_barrier();
+    auto block = [&](uint32_t u, const uint8_t (&act)[32][kRun], const float4 (&scl)[NT],
+                     uint8_t (&act_next)[32][kRun], float4 (&scl_next)[NT]) {
+        PairDecoder dec(w, h);
+        const uint32_t dw = h ? 0u : w.tl >> 16;  // the lane's row scale (binary16 bits) in half 0
+        if (u + 1 < nu) {
+            stage(u + 1, act_next, scl_next);
+            if (active) load_block_codes(rw, (u + 1) * trp * 28u, trp, row, w);
+        }
+        if (active) {
+            const float4 sg4 = scl[r32];
+            const float sg[4] = {sg4.x, sg4.y, sg4.z, sg4.w};
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const v16f dd = pinned_scale_products<HALF>(dw, sg[g], h);
+                uint32_t aw[4][2];
+                dec.group(g, aw);
+#pragma unroll
+                for (int l = 0; l < 4; ++l) {
+                    const v4h b = *reinterpret_cast<const v4h *>(&act[(4 * g + l) * 2 + h][r32 * 8]);
+                    const u32x2 a = {aw[l][0], aw[l][1]};
+                    const v16f i = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, a), b, zero, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) L[l][r] = __builtin_fmaf(i[r], dd[r], L[l][r]);
+                }
+            }
+        }
+        wait_vmcnt0();
+        lds_barrier();
+    };
+    for (uint32_t u = 0; u < nu; u += 2) {
+        block(u, act0, scl0, act1, scl1);
+        if (u + 1 < nu) block(u + 1, act1, scl1, act0, scl0);
+    }
+    pinned_store(L, active, t0 + r32, M, out + static_cast<size_t>(t0 + r32) * rows + static_cast<size_t>(tile) * kTile,
+                 out0, trows, err);
+}
+
 // The pinned contract (dot_q8_groups_pinned, src/kernels.rs:1102-1147): per (token, row) four
 // binary32 lanes L[l] = fma(I_l, dd_g, L[l]) with dd_g = fl(d_w * A_g.scale), group by group,
 // and (L0 + L1) + (L2 + L3) at the end.  In the pinned operand order one
@@ -609,12 +727,14 @@ struct LaneDecoder {
 // the two that share 32 rows decode half of them each (LaneDecoder) into LDS.  A block runs in
 // two halves of two groups, each half of the codes and of the operands in its own LDS buffer:
 // while one half is multiplied, the next half's codes stream into the other and its operands
-// are decoded into it, and one barrier a half hands both over (34 KiB, four workgroups a CU).
+// are decoded into it, and one barrier a half hands both over (50 KiB, three workgroups a CU).
+// A last group of at most 32 tokens would leave the second token wavefronts without products, so
+// it may take workgroups of 128 rows by 32 tokens (pinned_tail, the rule at the launch).
 template <bool HALF>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_prefill_ptq1_pinned(
     const uint8_t *W, uint32_t rows, uint32_t nu, const _Float16 *__restrict__ xh,
-    const float *__restrict__ sc, uint32_t M, uint32_t Mp, uint32_t xcd_major, float *__restrict__ out,
-    int *__restrict__ err) {
+    const float *__restrict__ sc, uint32_t M, uint32_t Mp, uint32_t form, uint32_t xcd_major,
+    float *__restrict__ out, int *__restrict__ err) {
     constexpr uint32_t NT = kPinnedTokens;
     constexpr uint32_t kRun = NT * 8;  // bytes of one (g, l, h) run of one block
     // Half 0: groups 0 and 1; half 1: groups 2 and 3.  act[4 (g % 2) + l][h][token][8 bytes],
@@ -632,7 +752,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const uint32_t hw = wave >> 1, tw = wave & 1;  // row half, token half
     const uint32_t tile = xcd_major ? blockIdx.y : blockIdx.x;
     const uint32_t by = xcd_major ? blockIdx.x + 8 * blockIdx.z : blockIdx.y;
-    const uint32_t t0 = by * NT, row_bytes = nu * 28;
+    const uint32_t t0 = by * (form == kPinnedAll32 ? NT / 2 : NT), row_bytes = nu * 28;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(xh, nu * 8u * Mp * 32u);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(sc, nu * Mp * 16u);
+    if (form == kPinnedAll32 || (form == kPinnedLast32 && M - t0 <= NT / 2)) {  // t0 < M: no empty groups in the grid
+        if (128 * tile < rows)
+            pinned_tail<HALF>(W, rows, nu, rx, rs, M, Mp, t0, tile, out, err, reinterpret_cast<uint8_t(&)[32][32 * 8]>(act0),
+                              reinterpret_cast<uint8_t(&)[32][32 * 8]>(act1), reinterpret_cast<float4(&)[32]>(scl0),
+                              reinterpret_cast<float4(&)[32]>(scl1));
+        return;
+    }
     const uint32_t left = rows - tile * kTile;  // tile * kTile < rows
     const uint32_t trows = left < kTile ? left : kTile, trp = (trows + 7u) & ~7u;
     // Uniform per wavefront: rows and tokens of its quarter exist.  The others still decode and
@@ -640,8 +769,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const bool active = 32 * hw < trows && t0 + 32 * tw < M;
     const __amdgpu_buffer_rsrc_t rw =
         make_rsrc(W + static_cast<size_t>(tile) * kTile * row_bytes, trp * row_bytes);
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(xh, nu * 8u * Mp * 32u);
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(sc, nu * Mp * 16u);
     const uint32_t row = 32 * hw + r32, out0 = 32 * hw + 4 * h;  // tile rows
 
     // Half `half` of block u's codes: 16 runs of NT * 8 bytes, each contiguous in xh and in LDS;
@@ -693,15 +820,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                         const u32x4 (&opa)[2][2][2][2][32]) {
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            // dd[r] = fl(d_w * A_g.scale) for every (row, token) of the tile, as an outer
-            // product: HALF where this library's quantizer made the scales, which are binary16
-            // values then; a caller's own blocks may hold any binary32 scale (K = 2 with the
-            // second term zero, one rounding).
-            v16f dd;
-            if constexpr (HALF)
-                dd = scale_products(da, h ? 0u : __builtin_bit_cast(uint16_t, static_cast<_Float16>(sg[g])));
-            else
-                dd = __builtin_amdgcn_mfma_f32_32x32x2f32(h2f(da), h ? 0.0f : sg[g], zero, 0, 0, 0);
+            const v16f dd = pinned_scale_products<HALF>(da, sg[g], h);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const u32x4 a2 = opa[hw][g][j][h][r32];  // native lanes j and j + 2
@@ -774,23 +893,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
     wait_vmcnt0();  // loads past the row's end still write LDS
     const uint32_t t = t0 + 32 * tw + r32;
-    if (!active || t >= M) return;
-    bool bad = false;
-    float *yr = out + static_cast<size_t>(t) * rows + static_cast<size_t>(tile) * kTile;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t r = out0 + 8 * q + e;
-            if (r < trows) {
-                const int k = 4 * q + e;
-                const float v = (L[0][k] + L[1][k]) + (L[2][k] + L[3][k]);
-                yr[r] = v;
-                bad |= !finite(v);
-            }
-        }
-    }
-    if (bad) raise_error(err, kErrNonfinite);
+    pinned_store(L, active, t, M, out + static_cast<size_t>(t) * rows + static_cast<size_t>(tile) * kTile, out0, trows, err);
 }
 
 uint32_t padded_tokens(uint32_t M) { return (M + kTokAlign - 1) / kTokAlign * kTokAlign; }
@@ -861,11 +964,32 @@ static int launch_ptq1(const void *w_tiled, uint64_t cols, uint64_t rows, const 
     const auto W = static_cast<const uint8_t *>(w_tiled);
     const uint32_t R = static_cast<uint32_t>(rows), nu = K / 128;
     if (pinned) {
-        const uint32_t groups = (M + kPinnedTokens - 1) / kPinnedTokens;  // token groups holding real tokens
-        const uint32_t tiles = static_cast<uint32_t>((rows + kTile - 1) / kTile);
-        const uint32_t xcd_major = groups % 8 == 0 && tiles <= 65535;
+        // Where the tokens end in the first half of a group of 64, two of its workgroups' four
+        // wavefronts would have no products, so it takes 128 x 32 workgroups where that takes one
+        // off the fullest CU or the grid does not run at once (three a CU).  Measured (us, 64 x 64
+        // throughout / last group 128 x 32; 128 x 32 throughout without the shared decode): 20000 x
+        // 4096, 65 tokens 82.0 / 62.9; 71.0, 17408 x 5120, 72 tokens 99.6 / 75.5; 86.3, 60000 x
+        // 2432, 32 tokens 68.9 / 42.2; 45.9, 24302 x 512, 463 tokens 67.0 / 61.4; 62.4, and with two
+        // a CU either way 4096 x 14336, 333 tokens 196 / 200; 225.  Rows of under eight blocks
+        // whose 128 x 32 workgroups all run at once take them throughout, the pipeline of the
+        // others being hardly filled when the row ends (8065 x 512, 203 tokens 18.2, here 16.5).
+        const uint64_t n32 = (M + 31) / 32, tiles64 = (rows + kTile - 1) / kTile;
+        const auto per_cu = [&](uint64_t workgroups) { return (workgroups + cus - 1) / cus; };
+        uint32_t form = kPinnedAll64;
+        if (n32 % 2) {
+            if (nu < 8 && gx * n32 <= 3ull * cus)
+                form = kPinnedAll32;
+            else if (const uint64_t all64 = per_cu(tiles64 * (n32 / 2 + 1));
+                     all64 > 3 || per_cu(tiles64 * (n32 / 2) + gx) < all64)
+                form = kPinnedLast32;
+        }
+        const uint32_t groups = static_cast<uint32_t>(form == kPinnedAll32 ? n32 : (n32 + 1) / 2);  // holding real tokens
+        const uint32_t tiles = form == kPinnedAll32 ? gx : static_cast<uint32_t>(tiles64);
+        // Token groups by XCD; not with a half one, whose XCD would idle while the others take more.
+        const uint32_t xcd_major = groups % 8 == 0 && form != kPinnedLast32 && tiles <= 65535;
         const dim3 grid = xcd_major ? dim3(8, tiles, groups / 8) : dim3(tiles, groups);
-        hipLaunchKernelGGL(k_prefill_ptq1_pinned<!BLOCKS>, grid, dim3(256), 0, s, W, R, nu, xh, sc, M, Mp, xcd_major, out, err);
+        hipLaunchKernelGGL(k_prefill_ptq1_pinned<!BLOCKS>, grid, dim3(256), 0, s, W, R, nu, xh, sc, M, Mp, form, xcd_major,
+                           out, err);
         return launch_status();
     }
     // Tokens per workgroup (measured, 6144 x 2048): 64 keeps three wavefronts per SIMD

@@ -62,3 +62,28 @@ def test_gpu_pinned_prefill_tiles_match_oracle(ctx, rows, cols, tokens):
     halves and token halves, and (513 tokens) a token half without tokens."""
     _check(ctx, ph.KIND_PTQ1, rows, cols, synth.ptq1_weights(rows, cols, seed=rows),
            synth.activations(cols, seed=tokens, tokens=tokens).reshape(tokens, cols), True, tokens)
+
+
+# The last group of at most 32 tokens on 128-row workgroups: alone, behind one, two and seven groups
+# of 64 (eight groups, of which seven are whole), its rows a partial tile, one tile of two, or two; and
+# short rows (under eight blocks) on those workgroups only, with the first of eight blocks beside them.
+@pytest.mark.parametrize("rows,cols,tokens", [(8192 + 37, 1280, 32), (8192 + 100, 1152, 65), (4096 + 64, 1664, 150),
+                                              (6144 + 31, 1152, 449), (8192 + 5, 896, 96), (8192 + 5, 1024, 96),
+                                              (8192 + 97, 256, 32)])
+@pytest.mark.parametrize("prepared", [False, True])
+def test_gpu_pinned_prefill_half_group_matches_oracle(ctx, rows, cols, tokens, prepared):
+    import oracle
+
+    w = synth.ptq1_weights(rows, cols, seed=rows)
+    X = synth.activations(cols, seed=tokens, tokens=tokens).reshape(tokens, cols)
+    if not prepared:
+        return _check(ctx, ph.KIND_PTQ1, rows, cols, w, X, True, tokens)
+    act = np.concatenate([oracle.quantize_q8_0(X[t], 2) for t in range(tokens)])
+    ref = oracle.prefill(ph.KIND_PTQ1, cols, rows, w, X, True, threads=THREADS)
+    wid = ctx.weight(ph.KIND_PTQ1, cols, rows, w)
+    try:
+        got = ctx.project_q8(wid, rows, act.view(ph.Q8_DTYPE), tokens=tokens, pinned=True)
+        g, r = (np.ascontiguousarray(a, np.float32).reshape(-1).view(np.uint32) for a in (got, ref))
+        assert np.array_equal(g, r), int((g != r).sum())
+    finally:
+        ctx.release(wid)
