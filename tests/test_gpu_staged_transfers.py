@@ -57,16 +57,69 @@ def test_gpu_staged_ffn_residual(tokens):
         assert np.array_equal(again.view(np.uint32), got.view(np.uint32))
 
 
-def test_gpu_pinned_host_arrays_transfer_directly():
-    cols, rows, tokens = 2048, 300, 200
+def _pinned(shape):
+    p = ctypes.c_void_p()
+    assert hip().hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(int(np.prod(shape)) * 4), 0) == 0
+    return p, np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), shape)
+
+
+@pytest.mark.parametrize("tokens", [300, 1100])  # 2.5 MB each way, below the slots' line; 9.0 and 9.2 MB
+def test_gpu_pinned_host_arrays_transfer_directly(tokens):
+    """Pinned input and output of a call give the pageable call's bits (that they bypass the slots is
+    shown where the copies are written down, test_host_scratch.py)."""
+    cols, rows = 2048, 2100
     with ph.Context(0) as ctx:
         wid = ctx.weight(ph.KIND_Q2_K, cols, rows, synth.weights(ph.KIND_Q2_K, rows, cols, seed=1))
         X = np.ascontiguousarray(synth.activations(cols, seed=2, tokens=tokens).reshape(tokens, cols), np.float32)
         want = ctx.project_f32(wid, rows, X, tokens=tokens)
-        p = ctypes.c_void_p()
-        assert hip().hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(X.nbytes), 0) == 0
-        pinned = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), X.shape)
-        pinned[:] = X
-        got = ctx.project_f32(wid, rows, pinned, tokens=tokens)
-        assert np.array_equal(np.asarray(got).view(np.uint32), np.asarray(want).view(np.uint32))
-        hip().hipHostFree(p)
+        (px, x), (po, out) = _pinned(X.shape), _pinned((tokens, rows))
+        x[:] = X
+        for _ in range(2):
+            out[:] = 7
+            assert ph.lib().prism_hip_project_f32(ctx._h, wid, px, tokens, 0, po) == 0
+            assert np.array_equal(out.view(np.uint32), np.asarray(want).view(np.uint32))
+        for p in (px, po):
+            hip().hipHostFree(p)
+
+
+@pytest.mark.parametrize("memory", ["pinned", "pinned, null stream", "device"])
+@pytest.mark.parametrize("tokens", [256, 1030])  # the smallest residual of the side stream (1 MiB), and staged sizes
+@pytest.mark.parametrize("which", ["input", "residual"])
+def test_gpu_host_call_reads_behind_queued_work(memory, tokens, which):
+    """A pinned or device array filled by a copy queued on the context stream (or the null stream,
+    which the context stream orders itself with) behind some ten milliseconds of kernels is read
+    when its turn comes: same bits as the synchronized call."""
+    hidden, ffn = 1024, 1536
+    with ph.Context(0) as ctx:
+        g, u = (ctx.weight(ph.KIND_PTQ1, hidden, ffn, synth.ptq1_weights(ffn, hidden, seed=s)) for s in (1, 2))
+        d = ctx.weight(ph.KIND_PTQ1, ffn, hidden, synth.ptq1_weights(hidden, ffn, seed=3))
+        big = ctx.weight(ph.KIND_PTQ1, 2048, 20000, synth.ptq1_weights(20000, 2048, seed=6))
+        bx = DeviceBuffer.from_numpy(np.ascontiguousarray(synth.activations(2048, seed=7, tokens=512), np.float32))
+        bo = DeviceBuffer(20000 * 512 * 4)
+        X, R = (np.ascontiguousarray(synth.activations(hidden, seed=s, tokens=tokens).reshape(tokens, hidden), np.float32)
+                for s in (4, 5))
+        want = ctx.ffn_chain_tokens(g, u, d, hidden, X, residual=R)
+        src = X if which == "input" else R
+        dsrc = DeviceBuffer.from_numpy(src)
+        own, late = None, None
+        if memory == "device":
+            late = DeviceBuffer.from_numpy(np.zeros_like(src))
+            ptr, kind = late.ptr, 3
+        else:
+            own, late = _pinned(src.shape)
+            late[:] = 0
+            ptr, kind = own.value, 2
+        out = np.full((tokens, hidden), 7.0, np.float32)
+        ctx.project_device(big, ph.PATH_F32, bx, 512, False, bo)
+        assert ctx.sync() == 0
+        for _ in range(100):
+            ctx.project_device(big, ph.PATH_F32, bx, 512, False, bo)
+        stream = None if memory.endswith("null stream") else ctx.stream()
+        assert hip().hipMemcpyAsync(ptr, dsrc.ptr, src.nbytes, kind, stream) == 0
+        px, pr = (ptr, R.ctypes.data) if which == "input" else (X.ctypes.data, ptr)
+        rc = ph.lib().prism_hip_ffn_chain_tokens(ctx._h, g, u, d, ctypes.c_void_p(px), ctypes.c_void_p(pr), tokens, 0, 0,
+                                                 ctypes.c_void_p(out.ctypes.data))
+        assert rc == 0
+        assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+        if own:
+            hip().hipHostFree(own)

@@ -82,6 +82,36 @@ def test_ffn_residual_is_copied_behind_the_callers_work(stub, memory):
         """, memory)
 
 
+@pytest.mark.parametrize("memory", ["pinned", "pageable"])
+@pytest.mark.parametrize("tokens,staged", [(300, False), (511, False), (512, True), (1100, True)])
+def test_large_pageable_arrays_pass_through_the_pinned_slots(stub, memory, tokens, staged):
+    """From 4 MiB a pageable array moves in pieces through pinned slots, allocated for the first such
+    call; a smaller one, and pinned memory of any size, in one copy of its own."""
+    stub("""
+        tokens, staged = int(sys.argv[4]), sys.argv[5] == "True" and sys.argv[3] == "pageable"
+        c = L.prism_hip_create(0, 0, 0)
+        w = weight(c, ph.KIND_Q2_K, 2048, 2048)
+        n = tokens * 2048 * 4
+        if sys.argv[3] == "pinned":
+            x, out = P(), P()
+            assert S.hipHostMalloc(ctypes.byref(x), n, 0) == 0 and S.hipHostMalloc(ctypes.byref(out), n, 0) == 0
+        else:
+            keep = [np.zeros(n // 4, np.float32) for _ in range(2)]
+            x, out = (P(a.ctypes.data) for a in keep)
+        log()
+        for call in range(2):
+            assert L.prism_hip_project_f32(c, w, x, tokens, 0, out) == 0
+            lines = log()
+            assert any(l.startswith("host_malloc") for l in lines) == (staged and call == 0), lines
+            sizes = [int(l.split()[4]) for l in lines if l.startswith("copy ") and int(l.split()[4]) > 4]
+            pieces = -(-n // (1536 * 1024))
+            assert len(sizes) == (2 * pieces if staged else 2) and sum(sizes) == 2 * n, lines
+            direct = sum(f"<- {hex(x.value)} {n} " in l or f"copy {hex(out.value)} " in l for l in lines)
+            assert direct == (0 if staged else 2), lines
+        L.prism_hip_destroy(c)
+        """, memory, tokens, staged)
+
+
 @pytest.mark.parametrize("seed", [1, 2])
 def test_a_call_made_once_uncaptured_can_be_captured(stub, seed):
     """Every form of a device call, at sizes on all routes: scratch never grows under capture, and one
