@@ -3609,11 +3609,17 @@ int launch_splitk(const MatvecArgs &a, uint32_t act_stride) {
 // / 38, 87 / 54; 4096 rows 160 (2560) 23 / 33, 46 / 49, 88 / 78, and a little lower up to 128
 // tokens, where the block-split kernel runs (2048 rows 100 tokens (896) 19 / 26, 35 / 34, 66 /
 // 48).
+// The skinny kernel's three launches (with the lane-ordered copy) against the GEMM's two lose on
+// short rows whatever their number: PQ2 20 x 256, 200 tokens 7.5 / 10.2, 1100 x 512, 120 tokens 8.7
+// / 10.2, 74 x 1024, 94 tokens 9.3 / 10.3; TQ1_0 50 x 512, 330 tokens 8.2 / 10.1, 3326 x 1024, 106
+// tokens 11.4 / 12.3; Q8_0 1100 x 256, 300 tokens 8.9 / 10.5, 2910 x 512, 176 tokens 11.6 / 13.0.
+// From 1280 inputs (Q8_0 640) the copy pays.
 bool skinny_beats_gemm(const MatvecArgs &a) {
     if (a.act_format == kActF32 || a.tokens < 2 || a.tokens > 512 || a.w2 || a.residual || a.tile_best) return false;
     const uint64_t w = skinny_blocks(a.rows) * ((a.tokens + kBatchMax - 1) / kBatchMax);
     return dispatch(a, [&]<Op O>() {
                const uint64_t nu = a.cols / unit_weights<O>();
+               if (a.cols < (O == Op::Q8_0 ? 640u : 1280u) && skinny_plan<O>(a).sw) return 0;
                uint64_t most;  // per 256 CUs
                if constexpr (O == Op::PTQ1_PINNED) most = nu < 44 ? 600 + 25 * nu : 1700;
                else if constexpr (kind_of<O>() == kPTQ1) most = nu < 50 ? (a.tokens > 128 ? 40 : 30) * nu : 2000;

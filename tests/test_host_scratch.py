@@ -219,3 +219,32 @@ def test_scratch_of_a_captured_call_outlives_larger_calls(stub, kind, rows, cols
         L.prism_hip_destroy(c)
         assert S.stub_allocations() == empty - 1, (S.stub_allocations(), empty)  # and the error flag
         """, kind, rows, cols, tokens, pinned, path, more, ffn)
+
+
+# The kernels a call is made of, at the lines between two of them (kind, rows, cols, tokens, pinned,
+# path, the launches' kernels in order); where each line lies is measured, at the rule in the source.
+ROUTES = [
+    # Short rows whose skinny batch would copy its activations stay on the GEMM.
+    ("PQ2", 74, 1024, 94, False, "F32", "prefill prefill_kq"),
+    ("PQ2", 74, 1280, 94, False, "F32", "quantize sk_prep skinny"),
+    ("TQ1_0", 700, 1024, 106, False, "F32", "prefill prefill_kq"),
+    ("TQ1_0", 700, 1280, 106, False, "Q8K", "sk_prep skinny"),
+    ("Q8_0", 1100, 512, 120, False, "Q8", "prefill prefill_kq"),
+    ("Q8_0", 1100, 768, 120, False, "F32", "quantize sk_prep skinny"),
+    ("Q2_K", 1100, 256, 120, False, "F32", "quantize skinny"),
+]
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens,pinned,path,kernels", ROUTES)
+def test_dispatch_lines(stub, kind, rows, cols, tokens, pinned, path, kernels):
+    stub("""
+        kind, path = getattr(ph, "KIND_" + sys.argv[3]), getattr(ph, "PATH_" + sys.argv[8])
+        rows, cols, tokens = (int(a) for a in sys.argv[4:7])
+        c = L.prism_hip_create(0, 0, 0)
+        w = weight(c, kind, cols, rows)
+        log()
+        assert project(c, w, path, tokens, sys.argv[7] == "True") == 0
+        names = [l.split()[1] for l in log() if l.startswith("launch ")]
+        want = sys.argv[9].split()
+        assert len(names) == len(want) and all(k in n for k, n in zip(want, names)), names
+        """, kind, rows, cols, tokens, pinned, path, kernels)
