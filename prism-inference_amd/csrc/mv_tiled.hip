@@ -3648,6 +3648,18 @@ bool gemm_eligible(const MatvecArgs &a) {
 
 bool skinny_eligible(const MatvecArgs &a) {
     if (a.tokens < 2 || a.w2 || lut_batch_eligible(a) || quad_eligible(a) || quad_split_eligible(a)) return false;
+    if (a.rows < kSkinnyMinRows && (a.kind == kQ8_0 || a.kind == kTQ1_0)) {
+        // Two tokens of long rows stay on the one-token kernels, whose split spreads a row over
+        // lane groups, where the skinny kernel's few workgroups walk it with fourteen of sixteen
+        // tokens empty.  Measured on 50 to 1000 rows (us, token by token / skinny): Q8_0 f32 6144
+        // inputs 12.6 / 13.4, 8192 14.4 / 16.1, 17408 20 / 27 (5120 14.0 / 12.9), prepared 5120
+        // 8.3 / 8.4, 6144 8.9 / 9.7, 8192 9.4 / 12.3, three prepared tokens 14336 19.2 / 19.7, 17408
+        // 21.7 / 23.0; TQ1_0 f32 14336 18.5 / 15.9, 16384 17.0 / 19.0, 17408 19.2 / 18.8, prepared
+        // 14336 11.2 / 12.1, 16384 10.3 / 15.1, 17408 14.7 / 14.9.
+        const bool prepared = a.act_format != kActF32;
+        if (a.tokens == 2 && a.cols >= (a.kind == kQ8_0 ? 6144u : prepared ? 14336u : 16384u)) return false;
+        if (a.tokens == 3 && a.kind == kQ8_0 && prepared && a.cols >= 14336) return false;
+    }
     if (a.rows < kSkinnyMinRows && a.act_format == kActF32) {
         // f32 input ran token by token here, each launch quantizing in its prologue: two
         // source-order PTQ1 tokens of rows too short for split-K stay there (us, token by token /

@@ -232,6 +232,16 @@ ROUTES = [
     ("Q8_0", 1100, 512, 120, False, "Q8", "prefill prefill_kq"),
     ("Q8_0", 1100, 768, 120, False, "F32", "quantize sk_prep skinny"),
     ("Q2_K", 1100, 256, 120, False, "F32", "quantize skinny"),
+    # Two (three) tokens of long rows on few rows stay on the one-token kernels.
+    ("Q8_0", 500, 6144, 2, False, "F32", "mv_split mv_split"),
+    ("Q8_0", 500, 5120, 2, False, "F32", "quantize skinny"),
+    ("Q8_0", 500, 6144, 2, False, "Q8", "mv_split mv_split"),
+    ("Q8_0", 500, 14336, 3, False, "Q8", "mv_split mv_split mv_split"),
+    ("Q8_0", 500, 14336, 3, False, "F32", "quantize sk_prep skinny"),
+    ("Q8_0", 1024, 14336, 2, False, "Q8", "sk_prep skinny"),
+    ("TQ1_0", 500, 16384, 2, False, "F32", "mv_split mv_split"),
+    ("TQ1_0", 500, 14336, 2, False, "F32", "quantize sk_prep skinny"),
+    ("TQ1_0", 500, 14336, 2, False, "Q8K", "mv_split mv_split"),
 ]
 
 
