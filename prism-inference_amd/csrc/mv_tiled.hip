@@ -3295,7 +3295,9 @@ size_t skinny_chunk_bytes(const MatvecArgs &a) {
 // 12.2, pinned 10.7 / 13.8, PQ2 4096 x 4096 10.0 / 10.8, TQ1_0 9.5 / 10.4; 16 tokens: PTQ1 850 x
 // 5120 20.9 / 17.8, PQ2 12.2 / 11.7, TQ1_0 12.4 / 11.4), from 5 where many units are gathered
 // (7 tokens: PTQ1 6144 x 5120 24.4 / 20.0, pinned 4302 x 10752 48.3 / 53.9, TQ1_0 1100 x 12800
-// 17.9 / 16.5), and not at all on short PTQ1 rows of few blocks (850 x 2560, 64 tokens 13.5 /
+// 17.9 / 16.5; PQ2 from 33 units, 1204 x 6784, 6 tokens 14.9 / 13.1, 2241 x 5760, 8 tokens 14.0 /
+// 12.1; seven and eight TQ1_0 tokens 4334 x 4096 13.4 / 11.8, 5947 x 5376 15.2 / 13.2), and not
+// at all on short PTQ1 rows of few blocks (850 x 2560, 64 tokens 13.5 /
 // 19.6, pinned 15.3 / 21.8; 2048 x 2048, 64 tokens 16.7 / 18.3, 96 tokens equal).  Every format
 // takes it from 8192 rows, but Q2_K's and TQ2_0's 256-element units halve the gathers (32768 x
 // 2048 Q2_K, 7 tokens 10.9 / 13.5; 40000 x 5120, 16 tokens 31.9 / 29.3).  PQ2 and Q8_0 rows of
@@ -3313,7 +3315,12 @@ SkinnyPlan skinny_plan(const MatvecArgs &a) {
     } else if (O == Op::Q8_0 || a.tokens <= 4) {
         pl.sw = a.tokens > 4;
     } else if (a.tokens <= 8) {
-        pl.sw = O == Op::TQ1 ? nu > 24 : blocks * nu > (O == Op::PTQ1_PINNED ? 96ull : 32ull) * a.cus;
+        if constexpr (O == Op::TQ1)
+            pl.sw = nu > 24 || (a.tokens > 6 && blocks * nu > 16ull * a.cus);
+        else if constexpr (kind_of<O>() == kPQ2)
+            pl.sw = nu > 32 || blocks * nu > 32ull * a.cus;
+        else
+            pl.sw = blocks * nu > (O == Op::PTQ1_PINNED ? 96ull : 32ull) * a.cus;
     } else {
         pl.sw = !(kind_of<O>() == kPTQ1 && nu <= 24 && a.rows < 4096 && blocks * chunks * nu <= 48ull * a.cus);
     }

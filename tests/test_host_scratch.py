@@ -242,6 +242,12 @@ ROUTES = [
     ("TQ1_0", 500, 16384, 2, False, "F32", "mv_split mv_split"),
     ("TQ1_0", 500, 14336, 2, False, "F32", "quantize sk_prep skinny"),
     ("TQ1_0", 500, 14336, 2, False, "Q8K", "mv_split mv_split"),
+    # Five to eight tokens copy their activations where many units would be gathered.
+    ("PQ2", 1204, 4096, 6, False, "F32", "quantize skinny"),
+    ("PQ2", 1204, 4352, 6, False, "F32", "quantize sk_prep skinny"),
+    ("TQ1_0", 4334, 4096, 6, False, "F32", "quantize skinny"),
+    ("TQ1_0", 4334, 4096, 7, False, "F32", "quantize sk_prep skinny"),
+    ("TQ1_0", 4000, 4096, 7, False, "F32", "quantize skinny"),
 ]
 
 
