@@ -248,6 +248,17 @@ ROUTES = [
     ("TQ1_0", 4334, 4096, 6, False, "F32", "quantize skinny"),
     ("TQ1_0", 4334, 4096, 7, False, "F32", "quantize sk_prep skinny"),
     ("TQ1_0", 4000, 4096, 7, False, "F32", "quantize skinny"),
+    # Few rows between the skinny kernel and the GEMMs.
+    ("PTQ1", 1638, 3456, 95, False, "F32", "prefill_prep prefill_ptq1_split"),
+    ("PTQ1", 1500, 3456, 95, False, "F32", "quantize sk_prep skinny"),
+    ("PTQ1", 6231, 7168, 70, False, "F32", "prefill_prep prefill_ptq1"),
+    ("PTQ1", 627, 2560, 422, True, "F32", "prefill_prep prefill_ptq1_pinned"),
+    ("PTQ1", 627, 2560, 390, True, "F32", "quantize sk_prep skinny"),
+    ("Q2_K", 1692, 16384, 250, False, "F32", "prefill prefill_kq"),
+    ("Q2_K", 1692, 8192, 250, False, "F32", "quantize skinny"),
+    ("TQ1_0", 1056, 2304, 320, False, "F32", "prefill prefill_kq"),
+    ("TQ1_0", 1056, 4352, 320, False, "F32", "quantize sk_prep skinny"),
+    ("TQ2_0", 2699, 8192, 127, False, "F32", "prefill prefill_kq"),
 ]
 
 
