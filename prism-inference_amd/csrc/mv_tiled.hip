@@ -3667,7 +3667,8 @@ bool skinny_eligible(const MatvecArgs &a) {
         // inputs 12.6 / 13.4, 8192 14.4 / 16.1, 17408 20 / 27 (5120 14.0 / 12.9), prepared 5120
         // 8.3 / 8.4, 6144 8.9 / 9.7, 8192 9.4 / 12.3, three prepared tokens 14336 19.2 / 19.7, 17408
         // 21.7 / 23.0; TQ1_0 f32 14336 18.5 / 15.9, 16384 17.0 / 19.0, 17408 19.2 / 18.8, prepared
-        // 14336 11.2 / 12.1, 16384 10.3 / 15.1, 17408 14.7 / 14.9.
+        // 14336 11.2 / 12.1, 16384 10.3 / 15.1, 17408 14.7 / 14.9.  f32 input below its own line is
+        // quantized first and then meets the line of prepared blocks.
         const bool prepared = a.act_format != kActF32;
         if (a.tokens == 2 && a.cols >= (a.kind == kQ8_0 ? 6144u : prepared ? 14336u : 16384u)) return false;
         if (a.tokens == 3 && a.kind == kQ8_0 && prepared && a.cols >= 14336) return false;

@@ -237,10 +237,11 @@ ROUTES = [
     ("Q8_0", 500, 5120, 2, False, "F32", "quantize skinny"),
     ("Q8_0", 500, 6144, 2, False, "Q8", "mv_split mv_split"),
     ("Q8_0", 500, 14336, 3, False, "Q8", "mv_split mv_split mv_split"),
-    ("Q8_0", 500, 14336, 3, False, "F32", "quantize sk_prep skinny"),
+    ("Q8_0", 500, 14336, 3, False, "F32", "quantize mv_split mv_split mv_split"),
     ("Q8_0", 1024, 14336, 2, False, "Q8", "sk_prep skinny"),
     ("TQ1_0", 500, 16384, 2, False, "F32", "mv_split mv_split"),
-    ("TQ1_0", 500, 14336, 2, False, "F32", "quantize sk_prep skinny"),
+    ("TQ1_0", 500, 12288, 2, False, "F32", "quantize skinny"),
+    ("TQ1_0", 500, 14336, 2, False, "F32", "quantize mv_split mv_split"),
     ("TQ1_0", 500, 14336, 2, False, "Q8K", "mv_split mv_split"),
     # Five to eight tokens copy their activations where many units would be gathered.
     ("PQ2", 1204, 4096, 6, False, "F32", "quantize skinny"),
