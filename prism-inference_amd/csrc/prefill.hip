@@ -973,10 +973,16 @@ static int launch_ptq1(const void *w_tiled, uint64_t cols, uint64_t rows, const 
         // a CU either way 4096 x 14336, 333 tokens 196 / 200; 225.  Rows of under eight blocks
         // whose 128 x 32 workgroups all run at once take them throughout, the pipeline of the
         // others being hardly filled when the row ends (8065 x 512, 203 tokens 18.2, here 16.5).
+        // Prepared blocks, whose binary32 scale products take VALU time, take them on rows of under
+        // thirteen blocks and up to one a CU (64 x 64 / 128 x 32: 13817 x 9728, 51 tokens 129 / 120,
+        // 3711 x 14976, 138 tokens 194 / 181, 12064 x 512, 360 tokens 33.1 / 30.8, 30580 x 1152, 121
+        // tokens 49.2 / 46.2; longer rows, more a CU 13234 x 4096, 297 tokens 144 / 150).
         const uint64_t n32 = (M + 31) / 32, tiles64 = (rows + kTile - 1) / kTile;
         const auto per_cu = [&](uint64_t workgroups) { return (workgroups + cus - 1) / cus; };
         uint32_t form = kPinnedAll64;
-        if (n32 % 2) {
+        if (BLOCKS && (nu < 13 || gx * n32 <= cus)) {
+            form = kPinnedAll32;
+        } else if (n32 % 2) {
             if (nu < 8 && gx * n32 <= 3ull * cus)
                 form = kPinnedAll32;
             else if (const uint64_t all64 = per_cu(tiles64 * (n32 / 2 + 1));
