@@ -854,7 +854,7 @@ static int ffn_checked(prism_hip_ctx *c, prism_weight_id gid, prism_weight_id ui
         rc = ffn_tokens_impl(c, *g, *u, d, static_cast<float *>(c->x.p),
                              residual ? static_cast<float *>(c->res.p) : nullptr, tokens, pinned,
                              static_cast<float *>(c->out.p), nullptr, c->stream, hb,
-                             beside ? std::function<int()>(residual_upload) : nullptr);
+                             beside ? std::function<int()>(std::ref(residual_upload)) : nullptr);  // ref: no allocation
     if (!rc) rc = finish(c, out, static_cast<float *>(c->out.p), nout);
     if (rc) {
         if (c->staging.side) (void)hipStreamSynchronize(c->staging.side);  // no upload outlives a failed call
