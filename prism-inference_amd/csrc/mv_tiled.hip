@@ -2916,7 +2916,9 @@ struct SplitPlan {
 // more lanes shorten it.  Measured (one token, f32 or prepared input as the dispatch has it,
 // us, 8 / 16): 5120 x 17408 PQ2 15.4 / 13.5, Q2_K 13.1 / 11.5, Q8_0 25.0 / 21.6, TQ1_0 15.9 /
 // 14.1; PTQ1, whose decode bounds it, loses (17.1 / 18.2), and so does a Q2_K prologue (15.1 /
-// 16.3: its workgroups quantize longer than they read).
+// 16.3: its workgroups quantize longer than they read).  Q8_0 between 10240 and 17408: 5243 x 11264
+// 16.8 / 16.1, 5909 x 13568 20.9 / 19.5, 13633 x 10368 27.7 / 25.0, 14147 x 14464 43.4 / 39.4 (just
+// above half a tile per CU 8400 x 13056 26.4 / 27.5).
 // max_lpr caps the lane groups per row (a workgroup then owns at least 64/max_lpr rows).
 template <Op O>
 bool plan_split(uint64_t rows, uint32_t nu, uint32_t cols, bool quant, uint32_t nmat, uint32_t cus, SplitPlan *pl,
@@ -2984,11 +2986,14 @@ bool takes_stream(uint64_t tiles, uint32_t nu, uint32_t cus) {
 // above half a tile per CU, where prepared blocks run on the row-tile kernels, 12288 x 17408 PQ2
 // 21.2 / 20.5, Q2_K 21.8 / 20.0, Q8_0 40.1 / 37.2 but 12288 x 10240 PQ2 14.5 / 15.8, and PTQ1
 // rows of 36 to 55 units (12288 x 5120 10.8 / 9.2, 2048 inputs 5.4 / 7.6).  Fewer tiles gain
-// nothing (4096 x 10240 PQ2 7.8 / 8.9).
+// nothing (4096 x 10240 PQ2 7.8 / 8.9), nor does half a tile per CU exactly, whose two lane groups a
+// row make one workgroup a CU, each quantizing beside the others (8192 x 10240 PQ2 9.7 / 10.6, 12288
+// Q2_K 10.2 / 11.5, TQ1_0 11.0 / 11.8, TQ2_0 9.0 / 9.7; equal from 14336).  Over 65 to 127 tiles TQ2_0
+// gains as Q2_K does: 5556 x 10496 10.2 / 9.5, 4729 x 13056 12.8 / 10.7, 5572 x 16896 14.4 / 10.9.
 template <Op O>
 bool long_rows_prepared(uint64_t tiles, uint64_t cols, uint32_t cus) {
-    if (4 * tiles <= cus || tiles >= cus || O == Op::PTQ1_PINNED) return false;
-    const bool few = 2 * tiles <= cus;
+    if (4 * tiles <= cus || 2 * tiles == cus || tiles >= cus || O == Op::PTQ1_PINNED) return false;
+    const bool few = 2 * tiles < cus;
     if constexpr (kind_of<O>() == kPTQ1) return few ? cols >= 14336 : cols >= 36 * 128 && cols < 56 * 128;
     if constexpr (O == Op::Q8_0) return !few && cols >= 16384;
     if constexpr (O == Op::TQ1) return few && cols >= 10240;

@@ -260,6 +260,15 @@ ROUTES = [
     ("TQ1_0", 1056, 2304, 320, False, "F32", "prefill prefill_kq"),
     ("TQ1_0", 1056, 4352, 320, False, "F32", "quantize sk_prep skinny"),
     ("TQ2_0", 2699, 8192, 127, False, "F32", "prefill prefill_kq"),
+    # One token of long rows: its quantizer in the prologue, or a launch of its own.
+    ("PQ2", 8192, 10240, 1, True, "F32", "mv_split"),
+    ("PQ2", 8128, 10240, 1, True, "F32", "quantize mv_split"),
+    ("TQ2_0", 8192, 12288, 1, False, "F32", "mv_split"),
+    ("TQ2_0", 8000, 12288, 1, False, "F32", "quantize mv_split"),
+    ("PTQ1", 8192, 16384, 1, False, "F32", "mv_split"),
+    ("Q2_K", 8256, 16384, 1, False, "F32", "quantize mv_rowsn"),
+    ("Q2_K", 8256, 14336, 1, False, "F32", "mv_split"),
+    ("Q2_K", 4096, 16384, 1, False, "F32", "mv_split"),
 ]
 
 
