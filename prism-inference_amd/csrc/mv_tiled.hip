@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(kLutThreads) void k_mv_rows_lut(MvParams p, const v
 // fold is as long as its dots); the single-term orders on the first.
 // kStreamRow: floats per term, the 64 rows and (pinned) 16 of padding, so that the two packed
 // words a wavefront's quads read lie in different banks.  The table, the buffers and the block
-// scales of 256 units take 157 KiB.
+// scales of 256 units take 158 KiB.
 constexpr uint32_t kStreamMaxUnits = 256;
 template <Op O>
 constexpr uint32_t kStreamRow = O == Op::PTQ1_PINNED ? 80 : 64;
@@ -3630,6 +3630,8 @@ int launch_splitk(const MatvecArgs &a, uint32_t act_stride) {
 // / 10.2, 74 x 1024, 94 tokens 9.3 / 10.3; TQ1_0 50 x 512, 330 tokens 8.2 / 10.1, 3326 x 1024, 106
 // tokens 11.4 / 12.3; Q8_0 1100 x 256, 300 tokens 8.9 / 10.5, 2910 x 512, 176 tokens 11.6 / 13.0.
 // From 1280 inputs (Q8_0 640) the copy pays.
+// Calls with a residual (an FFN's down projection) keep the GEMM and its separate addition: these
+// lines were measured without one.
 bool skinny_beats_gemm(const MatvecArgs &a) {
     if (a.act_format == kActF32 || a.tokens < 2 || a.tokens > 512 || a.w2 || a.residual || a.tile_best) return false;
     const uint64_t w = skinny_blocks(a.rows) * ((a.tokens + kBatchMax - 1) / kBatchMax);

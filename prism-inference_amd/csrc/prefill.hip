@@ -919,8 +919,11 @@ size_t prefill_scratch_bytes(uint32_t kind, uint64_t cols, uint32_t tokens) {
 // by side, each unit decoded once per chunk); few rows stay there longer (skinny_beats_gemm).  Measured (f32 input
 // with its quantization, GEMM / skinny, us): 16 tokens 6144 x 2048 18.9 / 13.9, 12288 x 4096
 // 30.2 / 20.9, 151936 x 4096 139 / 93; 32 tokens source 6144 x 2048 20.0 / 17.3, 12288 x 4096
-// 31.6 / 31.8, 17408 x 5120 38.2 / 46.6, 32768 x 4096 41.7 / 54.8; pinned 6144 x 2048 31.6 /
-// 27.0, 12288 x 4096 56.7 / 73.7; 48 tokens source 6144 x 2048 20.3 / 21.4, pinned 32.3 / 42.4.
+// 31.6 / 31.8, 17408 x 5120 38.2 / 46.6, 32768 x 4096 41.7 / 54.8; 48 tokens 6144 x 2048 20.3 / 21.4;
+// pinned, 32 tokens on the GEMM against 31 on the skinny kernel 8192 x 2048 29.3 / 20.9, 12288 x 4096
+// 51.8 / 46.1, 17408 x 5120 61.9 / 72.2, 32768 x 4096 51.5 / 74.6, 151936 x 2048 74.7 / 149 (the
+// skinny kernel has gained more than the GEMM since the line was drawn; on the smallest of these
+// matrices it would now be ahead past it).
 static uint32_t ptq1_gemm_min_tokens(uint64_t rows) { return rows < 8192 ? 33 : 32; }
 
 bool prefill_supported(uint32_t kind, uint64_t cols, uint64_t rows, int pinned, uint32_t tokens) {
