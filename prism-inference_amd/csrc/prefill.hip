@@ -975,7 +975,9 @@ static int launch_ptq1(const void *w_tiled, uint64_t cols, uint64_t rows, const 
         // 2432, 32 tokens 68.9 / 42.2; 45.9, 24302 x 512, 463 tokens 67.0 / 61.4; 62.4, and with two
         // a CU either way 4096 x 14336, 333 tokens 196 / 200; 225.  Rows of under eight blocks
         // whose 128 x 32 workgroups all run at once take them throughout, the pipeline of the
-        // others being hardly filled when the row ends (8065 x 512, 203 tokens 18.2, here 16.5).
+        // others being hardly filled when the row ends (8065 x 512, 203 tokens 18.2, here 16.5; 6144 x
+        // 768, 256 tokens 20.8, 19.8), and of under four blocks always (32768 x 256, 64 tokens 16.1,
+        // 13.7; 24576 x 256, 256 tokens 29.4, 27.7).
         // Prepared blocks, whose binary32 scale products take VALU time, take them on rows of under
         // thirteen blocks and up to one a CU (64 x 64 / 128 x 32: 13817 x 9728, 51 tokens 129 / 120,
         // 3711 x 14976, 138 tokens 194 / 181, 12064 x 512, 360 tokens 33.1 / 30.8, 30580 x 1152, 121
@@ -983,12 +985,10 @@ static int launch_ptq1(const void *w_tiled, uint64_t cols, uint64_t rows, const 
         const uint64_t n32 = (M + 31) / 32, tiles64 = (rows + kTile - 1) / kTile;
         const auto per_cu = [&](uint64_t workgroups) { return (workgroups + cus - 1) / cus; };
         uint32_t form = kPinnedAll64;
-        if (BLOCKS && (nu < 13 || gx * n32 <= cus)) {
+        if (BLOCKS ? nu < 13 || gx * n32 <= cus : nu < 4 || (nu < 8 && gx * n32 <= 3ull * cus)) {
             form = kPinnedAll32;
         } else if (n32 % 2) {
-            if (nu < 8 && gx * n32 <= 3ull * cus)
-                form = kPinnedAll32;
-            else if (const uint64_t all64 = per_cu(tiles64 * (n32 / 2 + 1));
+            if (const uint64_t all64 = per_cu(tiles64 * (n32 / 2 + 1));
                      all64 > 3 || per_cu(tiles64 * (n32 / 2) + gx) < all64)
                 form = kPinnedLast32;
         }

@@ -290,6 +290,8 @@ def test_dispatch_lines(stub, kind, rows, cols, tokens, pinned, path, kernels):
 # 64 x 64 (64-row tiles by groups of 64), 128 x 32 throughout (128-row blocks by groups of 32), by XCD.
 @pytest.mark.parametrize("rows,cols,tokens,path,grid", [
     (20000, 4096, 65, "F32", "313 2 1"), (8192, 896, 96, "F32", "64 3 1"), (8192, 1024, 96, "F32", "128 2 1"),
+    (8192, 896, 128, "F32", "64 4 1"), (32768, 256, 64, "F32", "256 2 1"), (65536, 384, 256, "F32", "8 512 1"),
+    (65536, 512, 256, "F32", "1024 4 1"),
     (20000, 896, 160, "F32", "313 3 1"), (6144, 2048, 512, "F32", "8 96 1"), (6144, 2048, 449, "F32", "8 96 1"), (6200, 2048, 449, "F32", "97 8 1"),
     (13817, 9728, 51, "Q8", "108 2 1"), (20000, 4096, 64, "Q8", "313 1 1"), (16384, 4096, 64, "Q8", "128 2 1"),
     (12064, 512, 360, "Q8", "95 12 1"), (12064, 1536, 360, "Q8", "95 12 1"), (12064, 1664, 360, "Q8", "189 6 1")])
