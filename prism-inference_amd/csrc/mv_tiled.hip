@@ -3386,13 +3386,15 @@ int launch_skinny(const MatvecArgs &a, const SkinnyPlan &pl, const void *act, ui
     // Measured (us, wavefronts 1 / 2 / 4 / 8): Q2_K 12288 x 4096 7 tokens (three workgroups per
     // CU) 12.1 / 12.2 / 10.4 / 10.7, PQ2 20.3 / 18.5 / 13.9 / 12.8; 32768 x 2048 (eight) Q2_K
     // 13.9 / 14.6 / 14.4 / 15.6, Q8_0 17.5 / 19.4 / 20.0 / 21.4; 40000 x 5120 16 tokens (ten) Q2_K
-    // 31.9 / - / 29.4 / -, TQ2_0 29.8 / - / 26.7 / -; from sixteen one is ahead.  Pinned PTQ1's fold
+    // 31.9 / - / 29.4 / -, TQ2_0 29.8 / - / 26.7 / -; from sixteen one is ahead, and
+    // two chunks of four blocks a CU keep eight (source PTQ1 16384 x 5120, 17 tokens 37.7 with four,
+    // 36.2, 14336 inputs, 20 tokens 84.5, 79.6).  Pinned PTQ1's fold
     // is its larger part, and its terms leave one workgroup of eight to a CU: 512 x 2048 7 tokens
     // 16.1 / 16.7 / 12.4 / 10.6, 6144 x 2048 (1.5 per CU) 16.1 / 18.4 / 15.5 / 17.5, 9000 x 4096
     // (2.2) 28.3 / 35.3 / 36.7 / 38.8.
     const uint64_t blocks = skinny_blocks(a.rows), wgs = blocks * chunks;
     const int ks = O == Op::PTQ1_PINNED ? (wgs >= 2ull * a.cus ? 1 : wgs > a.cus ? 4 : 8)
-                                        : (wgs >= 16ull * a.cus ? 1 : wgs >= 8ull * a.cus ? 4 : 8);
+                                        : (wgs >= 16ull * a.cus ? 1 : wgs > 8ull * a.cus || blocks >= 8ull * a.cus ? 4 : 8);
     const dim3 grid(static_cast<uint32_t>(blocks), chunks), block(64 * ks);
     auto go = [&]<bool SWv>() {
         if (ks == 1) hipLaunchKernelGGL((k_mv_skinny<O, SWv, 1>), grid, block, 0, a.stream, p);

@@ -269,6 +269,11 @@ ROUTES = [
     ("Q2_K", 8256, 16384, 1, False, "F32", "quantize mv_rowsn"),
     ("Q2_K", 8256, 14336, 1, False, "F32", "mv_split"),
     ("Q2_K", 4096, 16384, 1, False, "F32", "mv_split"),
+    # Wavefronts of a skinny workgroup (the kernel's last template argument).
+    ("PTQ1", 16384, 5120, 17, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi8"),
+    ("PTQ1", 16448, 5120, 17, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi4"),
+    ("PTQ1", 32768, 5120, 7, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi4"),
+    ("PTQ1", 65536, 5120, 7, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi1"),
 ]
 
 
