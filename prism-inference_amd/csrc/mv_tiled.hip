@@ -3626,7 +3626,7 @@ int launch_splitk(const MatvecArgs &a, uint32_t act_stride) {
 // GEMM was ahead at PTQ1 1638 x 3456, 95 tokens (W 624) 25.7 / 27.9, 6231 x 7168, 70 (1960) 46.3 /
 // 50.7, pinned 627 x 2560, 422 (1080) 38.7 / 42.1, Q2_K 1692 x 16384, 250 (1728) 79.5 / 88.5, TQ1_0
 // 1056 x 2304, 320 (1360) 17.2 / 18.2, 3021 x 2304, 100 (1344) 16.1 / 17.1, TQ2_0 2699 x 8192, 127
-// (1376) 34.7 / 38.0.
+// (1376) 34.7 / 38.0, Q8_0 17408 x 16384, 17 (2176) 130.6 / 146.8 (14336 inputs 114.9 / 106.5).
 // The skinny kernel's three launches (with the lane-ordered copy) against the GEMM's two lose on
 // short rows whatever their number: PQ2 20 x 256, 200 tokens 7.5 / 10.2, 1100 x 512, 120 tokens 8.7
 // / 10.2, 74 x 1024, 94 tokens 9.3 / 10.3; TQ1_0 50 x 512, 330 tokens 8.2 / 10.1, 3326 x 1024, 106
@@ -3644,7 +3644,7 @@ bool skinny_beats_gemm(const MatvecArgs &a) {
                if constexpr (O == Op::PTQ1_PINNED) most = nu < 44 ? 540 + 23 * nu : 1550;
                else if constexpr (kind_of<O>() == kPTQ1) most = nu < 50 ? (a.tokens > 128 ? 36 : 22) * nu : 1700;
                else if constexpr (O == Op::Q2K) most = nu < 48 ? 1900 : 1600;
-               else if constexpr (O == Op::Q8_0) most = 2400;
+               else if constexpr (O == Op::Q8_0) most = nu < 128 ? 2400 : 2000;
                else if constexpr (kind_of<O>() == kPQ2) most = 1300;
                else if constexpr (O == Op::TQ1) most = nu < 16 ? 1100 : 1400;
                else most = 1350;

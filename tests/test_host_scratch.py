@@ -274,6 +274,9 @@ ROUTES = [
     ("PTQ1", 16448, 5120, 17, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi4"),
     ("PTQ1", 32768, 5120, 7, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi4"),
     ("PTQ1", 65536, 5120, 7, False, "F32", "quantize sk_prep skinnyILNS0_2OpE0ELb1ELi1"),
+    # Long Q8_0 rows beside the GEMM.
+    ("Q8_0", 17408, 16384, 17, False, "F32", "prefill prefill_kq"),
+    ("Q8_0", 17408, 14336, 17, False, "F32", "quantize sk_prep skinny"),
 ]
 
 
