@@ -843,7 +843,7 @@ static int ffn_checked(prism_hip_ctx *c, prism_weight_id gid, prism_weight_id ui
     const bool beside = residual && tokens > 1 && rbytes >= kSideMin && pageable(residual) && staging_ready(c);
     auto residual_upload = [&]() -> int {
         Staging &st = c->staging;
-        const int urc = upload(c, c->res.p, residual, rbytes, st.side, "upload residual", 0);
+        const int urc = staged_upload(c, c->res.p, residual, rbytes, st.side, "upload residual");
         if (urc) return urc;
         HIP_OR_FAIL(c, hipEventRecord(st.side_done, st.side));
         HIP_OR_FAIL(c, hipStreamWaitEvent(c->stream, st.side_done, 0));

@@ -356,13 +356,8 @@ inline bool pageable(const void *p) {
 // (2.7 / 5.7 / 8.2 MB each way) took 469 / 838 / 1089 us, staged 464 / 748 / 988, and 200 tokens
 // 327 / 352; 512 KiB pieces gained nothing at 2.7 MB (394 / 422).  The array is read before the
 // call returns.
-inline int upload(prism_hip_ctx *c, void *dev, const void *host, size_t bytes, hipStream_t s, const char *what,
-                  size_t least = kStageMin) {
+inline int staged_upload(prism_hip_ctx *c, void *dev, const void *host, size_t bytes, hipStream_t s, const char *what) {
     hipError_t e = hipSuccess;
-    if (bytes < least || !pageable(host) || !staging_ready(c)) {
-        e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-        return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
-    }
     Staging &st = c->staging;
     for (size_t at = 0; at < bytes && e == hipSuccess; at += kStageBytes) {
         const size_t n = bytes - at < kStageBytes ? bytes - at : kStageBytes;
@@ -375,6 +370,13 @@ inline int upload(prism_hip_ctx *c, void *dev, const void *host, size_t bytes, h
         if (e == hipSuccess) e = hipEventRecord(st.done[k], s);
     }
     return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
+}
+inline int upload(prism_hip_ctx *c, void *dev, const void *host, size_t bytes, hipStream_t s, const char *what) {
+    if (bytes < kStageMin || !pageable(host) || !staging_ready(c)) {
+        const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+        return e == hipSuccess ? PRISM_OK : hip_fail(c, e, what);
+    }
+    return staged_upload(c, dev, host, bytes, s, what);
 }
 // The other way; the host array is complete when the call returns (or, not staged, when the
 // stream drains).

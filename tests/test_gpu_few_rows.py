@@ -128,3 +128,35 @@ def test_gpu_first_call_under_capture(kind, rows, cols, tokens, pinned):
             g.launch()
             assert d.sync() == 0
             assert np.array_equal(a.to_numpy(np.uint32), b.to_numpy(np.uint32))
+
+
+@pytest.mark.parametrize("kind,rows,cols,tokens,pinned", [
+    (ph.KIND_PTQ1, 8200, 5120, 1, False),  # a quantizer of its own: one token
+    (ph.KIND_PTQ1, 8256, 4096, 1, True),  # the stream form: one token
+    (ph.KIND_PTQ1, 2048, 2048, 7, True), (ph.KIND_Q8_0, 500, 2048, 12, True)])  # few rows, gathered and copied
+def test_gpu_replay_after_a_larger_call(kind, rows, cols, tokens, pinned):
+    """A captured call's scratch outlives larger calls of its context (tests/test_host_scratch.py shows
+    that its buffers are kept): replays before and after one give the uncaptured call's bits."""
+    import hiprt
+
+    X = np.ascontiguousarray(synth.activations(cols, seed=11, tokens=300).reshape(300, cols), np.float32)
+    with ph.Context(0) as c:
+        w = c.weight(kind, cols, rows, synth.weights(kind, rows, cols, seed=12))
+        x, a, b = DeviceBuffer.from_numpy(X), DeviceBuffer(rows * 300 * 4), DeviceBuffer(rows * tokens * 4)
+        c.project_device(w, ph.PATH_F32, x, tokens, pinned, b)
+        assert c.sync() == 0
+        want = b.to_numpy(np.uint32)
+        g = hiprt.Graph(c.stream(), lambda: c.project_device(w, ph.PATH_F32, x, tokens, pinned, b))
+        for larger in (0, 40, 300):
+            if larger:
+                c.project_device(w, ph.PATH_F32, x, larger, pinned, a)
+                assert c.sync() == 0
+            for _ in range(2):
+                b.zero()
+                g.launch()
+                assert c.sync() == 0
+                assert np.array_equal(b.to_numpy(np.uint32), want)
+        c.project_device(w, ph.PATH_F32, x, 300, pinned, a)
+        assert c.sync() == 0
+        assert np.array_equal(a.to_numpy(np.uint32)[:rows * tokens], want)
+        del g
