@@ -79,6 +79,8 @@ bool tiled_needs_prepared(const MatvecArgs &a);
 bool tiled_prologue_fits(const MatvecArgs &a);
 // Device scratch a tiled call needs (the lane-ordered activations of a skinny batch).
 size_t tiled_scratch_bytes(const MatvecArgs &a);
+// What the prefill GEMM would need for a call it covers (0: it does not), whichever kernel runs it.
+size_t tiled_gemm_bytes(const MatvecArgs &a);
 // Whether a call on prepared blocks whose token count the prefill GEMMs take is faster as a
 // skinny batch, with the scratch it has (scratch_fit).
 bool skinny_beats_gemm(const MatvecArgs &a);

@@ -3658,13 +3658,15 @@ bool skinny_beats_gemm(const MatvecArgs &a) {
 // prefill.hip).  Measured, 151936 x 4096, 16 tokens, us, skinny -> GEMM: Q2_K 79.6 -> 71.4,
 // Q8_0 167.8 -> 136.4.  Not with a residual, and not when the caller's scratch cannot hold the
 // token codes.
-bool gemm_eligible(const MatvecArgs &a) {
+static bool gemm_covers(const MatvecArgs &a) {
     if (a.act_format == kActF32 || a.w2 || a.residual || a.tile_best || a.tokens < 2) return false;
     const bool fits = a.act_format == kActQ8K
                           ? a.kind == kQ2_K || a.kind == kPQ2 || a.kind == kTQ1_0 || a.kind == kTQ2_0
                           : a.kind == kQ8_0 || a.kind == kPTQ1;
-    return fits && prefill_supported(a.kind, a.cols, a.rows, a.pinned, a.tokens) && !skinny_beats_gemm(a) &&
-           prefill_scratch_bytes(a.kind, a.cols, a.tokens) <= a.scratch_cap;
+    return fits && prefill_supported(a.kind, a.cols, a.rows, a.pinned, a.tokens);
+}
+bool gemm_eligible(const MatvecArgs &a) {
+    return gemm_covers(a) && !skinny_beats_gemm(a) && prefill_scratch_bytes(a.kind, a.cols, a.tokens) <= a.scratch_cap;
 }
 
 bool skinny_eligible(const MatvecArgs &a) {
@@ -3792,6 +3794,10 @@ size_t tiled_scratch_bytes(const MatvecArgs &a) {
         return 0;
     });
     return bytes;
+}
+
+size_t tiled_gemm_bytes(const MatvecArgs &a) {
+    return gemm_covers(a) && !token_by_token(a) ? prefill_scratch_bytes(a.kind, a.cols, a.tokens) : 0;
 }
 
 bool tiled_prologue_fits(const MatvecArgs &a) {

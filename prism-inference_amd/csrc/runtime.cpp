@@ -59,6 +59,12 @@ int project_f32_dev(prism_hip_ctx *c, const Weight &w, const float *x, uint32_t 
         return rc;
     }
     if (w.tiled) {
+        // As in run_matvec: a captured call of another token count may take the GEMM.
+        if (tokens >= kPrefillMinTokens && !scr.base && prefill_supported(w.kind, w.cols, w.rows, pinned, tokens)) {
+            const size_t pre = prefill_scratch_bytes(w.kind, w.cols, tokens);
+            if (pre > c->pre.cap && !capturing(c))
+                if (const int rc = ensure(c, c->pre, pre)) return rc;
+        }
         MatvecArgs a = f32_args(c, w, x, tokens, pinned, out, residual, s);
         bool prepared = tiled_needs_prepared(a);
         if (prepared) {

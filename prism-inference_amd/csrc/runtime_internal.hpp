@@ -481,6 +481,10 @@ inline int run_matvec(prism_hip_ctx *c, const MatvecArgs &args, bool tiled, Scra
             a.scratch_fit = scratch_room(c, sc, c->sk, need);
             if (a.scratch_fit < need) need = tiled_scratch_bytes(a);
         }
+        // A context's buffer is sized for the GEMM also where the skinny batch runs: a captured call
+        // of another token count may need as much (the GEMM's own, or split-K terms).
+        if (!(sc && sc->base))
+            if (const size_t gemm = tiled_gemm_bytes(a); gemm > need && gemm > c->sk.cap && !capturing(c)) need = gemm;
         if (need) {
             Scratch grow{c};
             const int e = (sc ? *sc : grow).get(c->sk, need, &a.scratch, &a.scratch_bytes);
